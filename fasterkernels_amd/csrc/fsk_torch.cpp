@@ -20,6 +20,8 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <utility>
+#include <vector>
 
 #include "fsk_decode.h"
 
@@ -421,6 +423,45 @@ void kv_write(const at::Tensor& k_in, const at::Tensor& v_in, const at::Tensor& 
   check(st);
 }
 
+// ---------------------------------------------------------------------------
+// e4m3 quantisation (fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16)
+// ---------------------------------------------------------------------------
+// (codes, scale) of each of 1 to 3 tensors of one dtype, in two launches.  The
+// codes keep a dense tensor's strides; other tensors are packed first.  Each
+// scale is a 0-dim fp32 device tensor.
+std::vector<std::pair<at::Tensor, at::Tensor>> quantize(const std::vector<at::Tensor>& xs, int64_t stream) {
+  if (xs.empty() || xs.size() > 3) raise(FSK_ERR_INVALID, "quantize takes 1 to 3 tensors");
+  on_gpu(xs[0], "x");
+  const c10::Device dev = xs[0].device();
+  const c10::DeviceGuard guard(dev);
+  const int n = (int)xs.size();
+  std::vector<at::Tensor> src;
+  std::vector<std::pair<at::Tensor, at::Tensor>> res;
+  const void* sp[3];
+  void* dp[3];
+  float* cp[3];
+  int64_t numel[3];
+  for (int i = 0; i < n; ++i) {
+    const at::Tensor& x = xs[i];
+    on_device(x, "x", dev);
+    if (x.scalar_type() != xs[0].scalar_type()) raise(FSK_ERR_INVALID, "the tensors must have one dtype");
+    const bool dense = x.is_non_overlapping_and_dense() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+    src.push_back(dense ? x : x.clone(at::MemoryFormat::Contiguous));
+    const at::Tensor codes = at::empty_like(src.back(), src.back().options().dtype(at::kFloat8_e4m3fn));
+    const at::Tensor sc = at::empty({}, x.options().dtype(at::kFloat));
+    sp[i] = src.back().data_ptr();
+    dp[i] = codes.data_ptr();
+    cp[i] = sc.data_ptr<float>();
+    numel[i] = x.numel();
+    res.emplace_back(codes, sc);
+  }
+  const int64_t nbytes = fsk_quantize_workspace_bytes(n);
+  const at::Tensor ws = workspace(nbytes, xs[0]);
+  check(fsk_quantize_e4m3(n, sp, numel, dtype_code(xs[0].scalar_type(), "x"), dp, cp, ws.data_ptr(), nbytes,
+                          stream_ptr(stream)));
+  return res;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_fsk_torch, m) {
@@ -448,6 +489,7 @@ PYBIND11_MODULE(_fsk_torch, m) {
   m.def("dense", &dense, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cache_lens"), py::arg("start_k_offsets"),
         py::arg("s_aux"), py::arg("q_scale"), py::arg("k_scale"), py::arg("v_scale"), py::arg("out_code"),
         py::arg("sink_mode"), py::arg("sm_scale"), py::arg("chunk_tokens"), py::arg("stream"));
+  m.def("quantize", &quantize, py::arg("tensors"), py::arg("stream"));
   m.def("kv_write", &kv_write, py::arg("k"), py::arg("v"), py::arg("k_pool"), py::arg("v_pool"), py::arg("slot_mapping"),
         py::arg("k_scale"), py::arg("v_scale"), py::arg("block_table"), py::arg("bt_updates"), py::arg("stream"));
 }

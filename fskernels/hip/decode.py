@@ -13,6 +13,7 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 from fasterkernels_amd import native as nat
 
@@ -47,16 +48,44 @@ def set_num_splits_fp8(n: int) -> None:
     _DECODE_NUM_SPLITS_FP8 = int(n)
 
 
+def _kernel_quantizes(x) -> bool:
+    """Whether quantize_to_fp8 may leave torch's operators: a plain fp32
+    tensor, and nothing active that records or transforms operators (it would
+    not see the kernels' launch)."""
+    return (type(x) is torch.Tensor and x.is_cuda and x.dtype is torch.float32
+            and not (x.requires_grad and torch.is_grad_enabled())
+            and not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x) and forward_ad._current_level < 0
+            and x.layout is torch.strided and x.numel() > 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
 def quantize_to_fp8(x: torch.Tensor):
     """Per-tensor e4m3 quantisation: scale = max|x| / 448 (floored at 1e-12/448).
 
     Same formula and return value as
     fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16: returns (x_fp8, scale)
-    with scale a 0-dim fp32 tensor on x's device.
+    with scale a 0-dim fp32 tensor on x's device.  Plain fp32 tensors on a GPU
+    take two launches of the library's kernels (the same scale and codes);
+    other tensors, and calls that torch records (autograd, tracing, functorch,
+    dispatch modes), the torch expression.
     """
+    if _kernel_quantizes(x):
+        return nat.ext().quantize([x], _stream(x))[0]
     scale = x.abs().max().clamp(min=1e-12) / FP8_MAX
     x_fp8 = (x / scale).clamp(-FP8_MAX, FP8_MAX).to(FP8_DTYPE)
     return x_fp8, scale
+
+
+def quantize_each_to_fp8(*tensors):
+    """``quantize_to_fp8(t.float())`` of up to three tensors, as one call:
+    f16, bf16 and fp32 GPU tensors of one dtype are read as they are (no fp32
+    copies) by two launches for all of them."""
+    first = tensors[0]
+    if first.dtype in (torch.float16, torch.bfloat16, torch.float32) and all(
+            t.dtype is first.dtype and t.is_cuda and t.numel() > 0 for t in tensors):
+        return nat.ext().quantize(list(tensors), _stream(first))
+    return [quantize_to_fp8(t.float()) for t in tensors]
 
 
 # ---------------------------------------------------------------------------

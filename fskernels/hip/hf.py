@@ -45,7 +45,7 @@ from typing import Optional, Tuple
 import torch
 
 from .decode import (_on_gpu, flash_decode_gqa_hf_dense_optimized, flash_decode_gqa_hf_fp8,
-                     quantize_to_fp8)
+                     quantize_each_to_fp8)
 
 try:  # captured before anything is patched, as the reference module does (:3)
     from transformers.models.qwen3.modeling_qwen3 import eager_attention_forward as _native_eager
@@ -123,16 +123,15 @@ def custom_hf_decode_attention_forward_fp8(module: torch.nn.Module, query_states
                                            key_states: torch.Tensor, value_states: torch.Tensor,
                                            attention_mask, scaling: float, dropout: float = 0.0, **kwargs):
     """FP8 variant: Q, K and V are quantised per call with per-tensor scales
-    (quantize_to_fp8, as triton_gqa_decode_hf_fp8.py:268-273 does) and decoded
-    by the e4m3 kernels; the output keeps the query dtype."""
+    (the codes of quantize_to_fp8 of their fp32 values, as
+    triton_gqa_decode_hf_fp8.py:268-273 takes them) and decoded by the e4m3
+    kernels; the output keeps the query dtype."""
     bounds = _decode_bounds(query_states, key_states, attention_mask, kwargs)
     if bounds is None:
         return native_eager_attention_forward(module, query_states, key_states, value_states,
                                               attention_mask, scaling, dropout, **kwargs)
     lens, starts = bounds
-    q8, sq = quantize_to_fp8(query_states.squeeze(2).float())
-    k8, sk = quantize_to_fp8(key_states.float())
-    v8, sv = quantize_to_fp8(value_states.float())
+    (q8, sq), (k8, sk), (v8, sv) = quantize_each_to_fp8(query_states.squeeze(2), key_states, value_states)
     out = flash_decode_gqa_hf_fp8(q8, k8, v8, lens, sq, sk, sv, query_states.dtype, start_k_offsets=starts,
                                   sm_scale=scaling)
     return out, None

@@ -342,6 +342,20 @@ FSK_API int fsk_debug_split(int64_t total, int chunk_min, int chunk_max,
                             int32_t *item_chunk, int32_t *item_slot,
                             int32_t *token_chunk);
 
+/* Per-tensor e4m3 quantisation of 1 to 3 tensors (an attention call's Q, K and
+ * V) in two launches.
+ * Replaces: fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16 (quantize_to_fp8).
+ * For each tensor of numel[i] contiguous elements of src_dtype (f16, bf16 or
+ * f32): scale[i] = max(max|x|, 1e-12) / 448 (fp32, device) and dst[i] =
+ * e4m3(clamp(x / scale[i], +-448)), computed in fp32.  A NaN in the tensor
+ * gives a NaN scale.  Pointers 16-byte aligned (scale: 4); the pointer arrays
+ * are read on the host before the call returns.  The workspace holds
+ * fsk_quantize_workspace_bytes(count) bytes, uninitialised. */
+FSK_API int64_t fsk_quantize_workspace_bytes(int count);
+FSK_API int fsk_quantize_e4m3(int count, const void *const *src, const int64_t *numel, int src_dtype,
+                      void *const *dst, float *const *scale,
+                      void *workspace, int64_t workspace_bytes, void *stream);
+
 /* Tuning knobs for benchmarking sweeps:
  *   "chunk_tokens"        fixed split size in tokens (0: chosen on the device)
  *   "waves_per_cu"        largest persistent grid, workgroups per CU (default

@@ -1919,7 +1919,7 @@ __global__ __launch_bounds__(kWriteThreads) void kv_write_kernel(WriteParams p) 
 // written once.  As torch operations this was eight passes over fp32 copies:
 // Q, K and V of 4 x 8 heads x 3827 tokens x 128 (bf16, 62.7 MB) in 24 launches,
 // 259 us; now the maxima take 13.2 us and the codes 17.1 us (traced), and the
-// fp8 attention call 81 us instead of 310.
+// fp8 attention call 45.6 us instead of 311 (with mask_bounds_kernel).
 constexpr int kQuantMax = 3;         // tensors per call
 constexpr int kQuantThreads = 256;
 constexpr int kQuantStep = 16;       // elements of a thread's step: one 16-byte store of codes
@@ -2093,6 +2093,124 @@ __global__ __launch_bounds__(kQuantThreads) void quant_codes_kernel(QuantParams 
     widen_at<kSrc>(t.src, tail, x[0]);
     t.dst[tail] = (uint8_t)codes4(x);
   }
+}
+
+// ---------------------------------------------------------------------------
+// Attended range of a decode step (the HF attention functions)
+// ---------------------------------------------------------------------------
+// [starts[b], ends[b]) of each sequence: the first and one past the last
+// attended position of the query's mask row, or from the step's position (and
+// a sliding window), in one launch.  Latency-bound: one workgroup per
+// sequence reads its row (4 KB at 2048 positions of bf16) with 16-byte loads,
+// all in flight at once, and reduces it in registers.  As nine torch kernels
+// (compare, arange, two selects, two reductions over int32 rows, ...) the
+// range cost more than the attention: 4 left-padded sequences of up to 2047
+// positions, attention call 64.3 us (host-bound), with this 2.4 us launch 15.7.
+constexpr int kBoundsThreads = 256;
+constexpr int kBool = FSK_BOOL;
+struct BoundsParams {
+  const uint8_t* mask;      // rows of S elements, or null
+  int64_t m_sb, m_ss;       // batch / position strides, bytes
+  const int64_t* position;  // without a mask: the step's position, or null (length S)
+  int64_t window;           // without a mask: attend the last `window` positions (< 0: all)
+  int B, S;
+  int32_t* ends;
+  int32_t* starts;          // or null (without a mask and window)
+};
+
+// Bit e: element e of the 16 bytes is attended (0 in a float mask, nonzero in a bool one).
+template <int kM>
+__device__ __forceinline__ uint32_t attended16(u32x4 w) {
+  uint32_t bits = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t x = w[i];
+    if constexpr (kM == kF32) {
+      bits |= ((x & 0x7fffffffu) == 0 ? 1u : 0u) << i;
+    } else if constexpr (kM == kBool) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bits |= ((x & (0xffu << (8 * e))) != 0 ? 1u : 0u) << (4 * i + e);
+    } else {
+      bits |= ((x & 0x7fffu) == 0 ? 1u : 0u) << (2 * i);
+      bits |= ((x & 0x7fff0000u) == 0 ? 1u : 0u) << (2 * i + 1);
+    }
+  }
+  return bits;
+}
+template <int kM>
+__device__ __forceinline__ bool attended(const uint8_t* p) {
+  if constexpr (kM == kF32) return (*(const uint32_t*)p & 0x7fffffffu) == 0;
+  else if constexpr (kM == kBool) return *p != 0;
+  else return (*(const uint16_t*)p & 0x7fffu) == 0;
+}
+
+template <int kM>
+__global__ __launch_bounds__(kBoundsThreads) void mask_bounds_kernel(BoundsParams p) {
+  constexpr int kSize = kM == kF32 ? 4 : kM == kBool ? 1 : 2;
+  constexpr int kE = 16 / kSize;  // elements of a 16-byte load
+  constexpr int kUnroll = 4;
+  const int b = blockIdx.x;
+  const uint8_t* row = p.mask + b * p.m_sb;
+  int first = p.S, end = 0;
+  auto take = [&](int i) {
+    if (attended<kM>(row + i * p.m_ss)) {
+      first = min(first, i);
+      end = max(end, i + 1);
+    }
+  };
+  if (p.m_ss == kSize) {
+    // 16-byte loads over the row's aligned part; the elements before and
+    // after it (rows of an odd length start anywhere), one a thread
+    const int pre = min(p.S, (int)((0 - (uintptr_t)row) & 15) / kSize);
+    const int n = (p.S - pre) / kE;
+    const u32x4* body = (const u32x4*)(row + pre * kSize);
+    const int edge = (int)threadIdx.x < pre ? (int)threadIdx.x : n * kE + (int)threadIdx.x;
+    if (edge < p.S) take(edge);
+    for (int i0 = threadIdx.x; i0 < n; i0 += kUnroll * kBoundsThreads) {
+      u32x4 w[kUnroll];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) w[u] = body[min(i0 + u * kBoundsThreads, n - 1)];
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const uint32_t bits = attended16<kM>(w[u]);
+        const int at = pre + min(i0 + u * kBoundsThreads, n - 1) * kE;  // (a repeated last load changes nothing)
+        if (bits) {
+          first = min(first, at + __builtin_ctz(bits));
+          end = max(end, at + 32 - __builtin_clz(bits));
+        }
+      }
+    }
+  } else {
+    for (int i = threadIdx.x; i < p.S; i += kBoundsThreads) take(i);
+  }
+  __shared__ int s_first[kBoundsThreads / kWave], s_end[kBoundsThreads / kWave];
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    first = min(first, __shfl_xor(first, o));
+    end = max(end, __shfl_xor(end, o));
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    s_first[threadIdx.x / kWave] = first;
+    s_end[threadIdx.x / kWave] = end;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+#pragma unroll
+  for (int i = 1; i < kBoundsThreads / kWave; ++i) {
+    first = min(first, s_first[i]);
+    end = max(end, s_end[i]);
+  }
+  p.ends[b] = end;
+  p.starts[b] = min(first, end);
+}
+
+// Without a mask: every sequence of the batch has the same range.
+__global__ __launch_bounds__(kBoundsThreads) void position_bounds_kernel(BoundsParams p) {
+  const int b = blockIdx.x * kBoundsThreads + threadIdx.x;
+  if (b >= p.B) return;
+  const int len = p.position ? (int)(*p.position + 1) : p.S;
+  p.ends[b] = len;
+  if (p.starts) p.starts[b] = (int)max((int64_t)len - p.window, (int64_t)0);
 }
 
 // ---------------------------------------------------------------------------
@@ -2841,6 +2959,39 @@ int run_quantize(int count, const void* const* src, const int64_t* numel, int sr
   return FSK_OK;
 }
 
+int run_bounds(const void* mask, int mask_dt, int64_t sb, int64_t ss, const int64_t* position, int64_t window, int B,
+               int S, int32_t* ends, int32_t* starts, hipStream_t stream) {
+  if (B < 0 || S <= 0) return fail(FSK_ERR_INVALID, "batch and positions must be positive");
+  if (B > kMaxBatch) return fail(FSK_ERR_UNSUPPORTED, "batch above 16384");
+  if (!ends || ((mask || window >= 0) && !starts)) return fail(FSK_ERR_INVALID, "null output pointer");
+  if (B == 0) return FSK_OK;
+  BoundsParams p;
+  memset(&p, 0, sizeof(p));
+  p.position = position; p.window = window;
+  p.B = B; p.S = S; p.ends = ends; p.starts = starts;
+  if (mask) {
+    if (position || window >= 0) return fail(FSK_ERR_INVALID, "a mask, or a position and window");
+    const int size = mask_dt == FSK_BOOL ? 1 : mask_dt == FSK_E4M3 ? 0 : elem_bytes(mask_dt);
+    if (size == 0) return fail(FSK_ERR_UNSUPPORTED, "the mask must be bool, f16, bf16 or f32");
+    if (sb < 0 || ss < 0) return fail(FSK_ERR_INVALID, "negative stride");
+    if (sb >= kMaxStride || ss >= kMaxStride) return fail(FSK_ERR_UNSUPPORTED, "stride above 2^40 elements");
+    if (!aligned(mask, size)) return fail(FSK_ERR_INVALID, "mask not aligned to its type");
+    p.mask = (const uint8_t*)mask;
+    p.m_sb = sb * size; p.m_ss = ss * size;
+  }
+  (void)hipGetLastError();
+  const Launch l{stream, nullptr, nullptr};
+  const dim3 grid((unsigned)B), block(kBoundsThreads);
+  if (!mask) launch(position_bounds_kernel, dim3((unsigned)cdiv(B, kBoundsThreads)), block, 0, l, p);
+  else if (mask_dt == FSK_BOOL) launch(mask_bounds_kernel<kBool>, grid, block, 0, l, p);
+  else if (mask_dt == FSK_F16) launch(mask_bounds_kernel<kF16>, grid, block, 0, l, p);
+  else if (mask_dt == FSK_BF16) launch(mask_bounds_kernel<kBF16>, grid, block, 0, l, p);
+  else launch(mask_bounds_kernel<kF32>, grid, block, 0, l, p);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(FSK_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(e));
+  return FSK_OK;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -2952,6 +3103,12 @@ int64_t fsk_workspace_bytes(int layout, int batch, int num_q_heads, int num_kv_h
                                   chunk_tokens, device_cus(), 2);
   const int64_t u_max = sp.u_max;
   return ws_layout(B, num_kv_heads, G, head_dim, u_max).total;
+}
+
+int fsk_decode_bounds(const void* mask, int mask_dtype, int64_t stride_b, int64_t stride_s, const int64_t* position,
+                      int64_t window, int batch, int num_positions, int32_t* ends, int32_t* starts, void* stream) {
+  return run_bounds(mask, mask_dtype, stride_b, stride_s, position, window, batch, num_positions, ends, starts,
+                    (hipStream_t)stream);
 }
 
 int64_t fsk_quantize_workspace_bytes(int count) {

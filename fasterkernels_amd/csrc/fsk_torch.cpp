@@ -17,6 +17,7 @@
 
 #include <c10/core/DeviceGuard.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <string>
@@ -424,6 +425,48 @@ void kv_write(const at::Tensor& k_in, const at::Tensor& v_in, const at::Tensor& 
 }
 
 // ---------------------------------------------------------------------------
+// Attended range of an HF decode step (fskernels.hip.hf)
+// ---------------------------------------------------------------------------
+// (ends, starts) int32 [B] for a batch of B sequences over S positions, from
+// the last query's row of a [B or 1, heads, queries, >= S] mask, else from the
+// last entry of cache_position (int64), else S, with an optional window
+// (starts is undefined without a mask and window).
+std::pair<at::Tensor, c10::optional<at::Tensor>> bounds(const at::Tensor& like, int64_t B, int64_t S,
+                                                        const c10::optional<at::Tensor>& mask,
+                                                        const c10::optional<at::Tensor>& position,
+                                                        c10::optional<int64_t> window, int64_t stream) {
+  on_gpu(like, "query_states");
+  const c10::Device dev = like.device();
+  const c10::DeviceGuard guard(dev);
+  const at::Tensor out = at::empty({2, B}, like.options().dtype(at::kInt));
+  int32_t* ends = out.data_ptr<int32_t>();
+  const void* mp = nullptr;
+  int md = FSK_F32;
+  int64_t sb = 0, ss = 0;
+  const int64_t* pp = nullptr;
+  if (mask && mask->defined()) {
+    on_device(*mask, "attention_mask", dev);
+    if (mask->dim() != 4 || mask->size(1) < 1 || mask->size(2) < 1 || (mask->size(0) != B && mask->size(0) != 1) ||
+        (mask->size(3) < S && mask->size(3) != 1))
+      raise(kRuntime, "attention_mask must be [" + std::to_string(B) + ", heads, queries, >= " + std::to_string(S) +
+                          "], got " + shape_str(*mask));
+    md = mask->scalar_type() == at::kBool ? FSK_BOOL : dtype_code(mask->scalar_type(), "attention_mask");
+    sb = mask->size(0) == 1 ? 0 : mask->stride(0);
+    ss = mask->size(3) == 1 ? 0 : mask->stride(3);
+    mp = static_cast<const char*>(mask->data_ptr()) + (mask->size(2) - 1) * mask->stride(2) * mask->element_size();
+  } else if (position && position->defined()) {
+    on_device(*position, "cache_position", dev);
+    if (position->scalar_type() != at::kLong || position->dim() != 1 || position->numel() < 1)
+      raise(FSK_ERR_INVALID, "cache_position must be a non-empty int64 vector");
+    pp = position->data_ptr<int64_t>() + (position->numel() - 1) * position->stride(0);
+  }
+  const bool with_starts = mp || window;
+  check(fsk_decode_bounds(mp, md, sb, ss, pp, !mp && window ? std::max<int64_t>(*window, 0) : -1, (int)B, (int)S, ends,
+                          with_starts ? ends + B : nullptr, stream_ptr(stream)));
+  return {out.select(0, 0), with_starts ? c10::optional<at::Tensor>(out.select(0, 1)) : c10::nullopt};
+}
+
+// ---------------------------------------------------------------------------
 // e4m3 quantisation (fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16)
 // ---------------------------------------------------------------------------
 // (codes, scale) of each of 1 to 3 tensors of one dtype, in two launches.  The
@@ -489,6 +532,8 @@ PYBIND11_MODULE(_fsk_torch, m) {
   m.def("dense", &dense, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("cache_lens"), py::arg("start_k_offsets"),
         py::arg("s_aux"), py::arg("q_scale"), py::arg("k_scale"), py::arg("v_scale"), py::arg("out_code"),
         py::arg("sink_mode"), py::arg("sm_scale"), py::arg("chunk_tokens"), py::arg("stream"));
+  m.def("bounds", &bounds, py::arg("like"), py::arg("batch"), py::arg("positions"), py::arg("mask"),
+        py::arg("cache_position"), py::arg("window"), py::arg("stream"));
   m.def("quantize", &quantize, py::arg("tensors"), py::arg("stream"));
   m.def("kv_write", &kv_write, py::arg("k"), py::arg("v"), py::arg("k_pool"), py::arg("v_pool"), py::arg("slot_mapping"),
         py::arg("k_scale"), py::arg("v_scale"), py::arg("block_table"), py::arg("bt_updates"), py::arg("stream"));

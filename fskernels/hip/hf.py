@@ -44,8 +44,12 @@ from typing import Optional, Tuple
 
 import torch
 
-from .decode import (_on_gpu, flash_decode_gqa_hf_dense_optimized, flash_decode_gqa_hf_fp8,
+from fasterkernels_amd import native as nat
+
+from .decode import (_on_gpu, _stream, flash_decode_gqa_hf_dense_optimized, flash_decode_gqa_hf_fp8,
                      quantize_each_to_fp8)
+
+_MASK_DTYPES = (torch.bool, torch.float16, torch.bfloat16, torch.float32)
 
 try:  # captured before anything is patched, as the reference module does (:3)
     from transformers.models.qwen3.modeling_qwen3 import eager_attention_forward as _native_eager
@@ -66,7 +70,7 @@ def _decode_bounds(query_states: torch.Tensor, key_states: torch.Tensor, attenti
                    kwargs) -> Optional[Tuple[torch.Tensor, Optional[torch.Tensor]]]:
     """(cache_lens, start_offsets) of a decode step, or None for other calls.
 
-    All values are computed on the device:
+    All values are computed on the device, in one launch:
     * with ``cache_position`` (transformers versions that pass it, and the
       reference's contract): length cache_position[-1] + 1 and, for a sliding
       window, start max(0, length - window);
@@ -81,9 +85,22 @@ def _decode_bounds(query_states: torch.Tensor, key_states: torch.Tensor, attenti
         return None
     _on_gpu(query_states, "query_states")
     S = key_states.shape[2]
-    dev = query_states.device
     window = kwargs.get("sliding_window")
     cache_position = kwargs.get("cache_position")
+    if cache_position is not None:
+        attention_mask = None
+        kernel = cache_position.dtype is torch.int64 and cache_position.dim() == 1 and cache_position.is_cuda
+    else:
+        kernel = attention_mask is None or (attention_mask.dtype in _MASK_DTYPES and attention_mask.dim() == 4)
+    if not kernel or not 0 < S < 1 << 31:
+        return _torch_bounds(bsz, S, query_states.device, attention_mask, cache_position, window)
+    return nat.ext().bounds(query_states, bsz, S, attention_mask, cache_position,
+                            None if window is None else int(window), _stream(query_states))
+
+
+def _torch_bounds(bsz, S, dev, attention_mask, cache_position, window):
+    """_decode_bounds in torch operations, for the mask and position types
+    that the kernel does not read (integer and fp64 masks, other positions)."""
     if cache_position is not None:
         lens = (cache_position[-1:] + 1).to(torch.int32).expand(bsz).contiguous()
     elif attention_mask is not None:

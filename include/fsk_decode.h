@@ -50,6 +50,7 @@ extern "C" {
 #define FSK_BF16 1
 #define FSK_F32 2
 #define FSK_E4M3 3 /* OCP float8 e4m3fn (torch.float8_e4m3fn) */
+#define FSK_BOOL 4 /* one byte, nonzero = true (fsk_decode_bounds' mask only) */
 
 /* Sink folding.  With s = q.k * sm_scale over the sequence and a per-q-head
  * sink value z:
@@ -341,6 +342,21 @@ FSK_API int fsk_debug_split(int64_t total, int chunk_min, int chunk_max,
                             int32_t *geometry, int32_t *chunk_start,
                             int32_t *item_chunk, int32_t *item_slot,
                             int32_t *token_chunk);
+
+/* Attended range [starts[b], ends[b]) of a decode step with one query
+ * position per sequence, for the dense entry point's start_offsets and
+ * cache_lens, in one launch.
+ * Replaces: fskernels/triton/triton_gqa_decode_hf.py:240-250 (lengths from the
+ * step's position, sliding window).
+ * With a mask (bool: nonzero = attended; f16, bf16, f32: zero = attended; row b
+ * at stride_b * b elements, num_positions elements stride_s apart): the first
+ * and one past the last attended position (both 0 if there is none); position
+ * is NULL and window negative.  Without: ends = *position + 1 (num_positions if
+ * position, a device int64, is NULL) and, if window >= 0, starts =
+ * max(0, ends - window) (else starts may be NULL). */
+FSK_API int fsk_decode_bounds(const void *mask, int mask_dtype, int64_t stride_b, int64_t stride_s,
+                      const int64_t *position, int64_t window, int batch, int num_positions,
+                      int32_t *ends, int32_t *starts, void *stream);
 
 /* Per-tensor e4m3 quantisation of 1 to 3 tensors (an attention call's Q, K and
  * V) in two launches.

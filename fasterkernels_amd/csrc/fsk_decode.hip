@@ -837,9 +837,10 @@ __device__ __forceinline__ LaneGeo<D, kKV> lane_geo(const Params& p, int lane, i
   return lg;
 }
 
-template <int D, int kKV, int kLayout>
-__device__ __forceinline__ void issue_tile(TileRegs<D, kKV>& T, uint32_t kstage_off, const Params& p,
-                                           const Unit& un, int t, const LaneGeo<D, kKV>& lg) {
+// half(h2): the addresses and valid rows of the tile's 16-row half h2.
+template <int D, int kKV, typename Half>
+__device__ __forceinline__ void issue_tile(TileRegs<D, kKV>& T, uint32_t kstage_off, const Params& p, Half half,
+                                           const LaneGeo<D, kKV>& lg) {
   using TR = TileRegs<D, kKV>;
   constexpr int kElem = TR::kFp8 ? 1 : 2;
   const int kst = (int)p.k_st, vst = (int)p.v_st;
@@ -847,7 +848,7 @@ __device__ __forceinline__ void issue_tile(TileRegs<D, kKV>& T, uint32_t kstage_
   asm volatile("" ::: "memory");
 #pragma unroll
   for (int h2 = 0; h2 < 2; ++h2) {
-    const HalfTile ht = unit_half<kLayout>(p, un, t + 16 * h2);
+    const HalfTile ht = half(h2);
     T.nrow[h2] = ht.rows;
     const int kbytes = ht.rows > 0 ? (ht.rows - 1) * kst + D * kElem : 0;
     const int vbytes = ht.rows > 0 ? (ht.rows - 1) * vst + D * kElem : 0;
@@ -1344,6 +1345,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
       }
     }
     BlockMax bm;
+    auto issue = [&](TR& T, int slot, int t) {
+      issue_tile<D, kKV>(T, s_kstage + slot * 2 * TR::kHalfBytes, p,
+                         [&](int h2) { return unit_half<kLayout>(p, un, t + 16 * h2); }, lg);
+    };
 
     if constexpr (kDepth > 1) {
       // Tile slot s holds tile n with n % kDepth == s (its K stage is slot s
@@ -1359,8 +1364,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
       int k = 0;  // tiles computed so far
 #pragma unroll
       for (int s = 0; s < kDepth - 1; ++s)
-        issue_tile<D, kKV, kLayout>(tiles[s], s_kstage + s * 2 * TR::kHalfBytes, p, un,
-                                    tile_pos(s, n_tiles, rot, un.t_begin, un.t_end), lg);
+        issue(tiles[s], s, tile_pos(s, n_tiles, rot, un.t_begin, un.t_end));
       bool done = false;
       while (!done) {
 #pragma unroll
@@ -1368,7 +1372,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
           if (!done) {
             const int tn = tile_pos(k + kDepth - 1, n_tiles, rot, un.t_begin, un.t_end);
             const int sn = (s + kDepth - 1) % kDepth;
-            issue_tile<D, kKV, kLayout>(tiles[sn], s_kstage + sn * 2 * TR::kHalfBytes, p, un, tn, lg);
+            issue(tiles[sn], sn, tn);
             wait_k_stage<TR::kLoads, kDepth>(kDepth - 1);
             if (k == 0 && segments_done == 0) FSK_STAMP(2);
             if constexpr (kValu) {
@@ -1386,7 +1390,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
     } else {
       TR ta;
       for (int t = un.t_begin; t < un.t_end; t += 32) {
-        issue_tile<D, kKV, kLayout>(ta, s_kstage, p, un, t, lg);
+        issue(ta, 0, t);
         wait_k_stage<TR::kLoads, 1>(0);
         if (t == un.t_begin && segments_done == 0) FSK_STAMP(2);
         if constexpr (kValu) {
@@ -1446,6 +1450,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
   FSK_STAMP(4);
   (void)segments_done;
   (void)hp;
+}
+
+// The sink folded into a row's denominator (M: the row's maximum score, log2
+// domain; den: its sum of exponentials relative to M): the new denominator,
+// the factor of the numerator (exp sinks) and the reference point of both.
+struct SinkFold {
+  float den, fs, ref;
+};
+__device__ __forceinline__ SinkFold fold_sink(float M, float den, bool sink, int mode, float z) {
+  const float M_use = (M == -INFINITY) ? 0.f : M;
+  SinkFold f{den, 1.f, M_use};
+  if (!sink) return f;
+  if (mode == FSK_SINK_EXP) {
+    // Extra logit z with a zero value vector (log2 domain: z * log2 e).
+    const float z2 = z * kLog2e;
+    const float Mn = fmaxf(M, z2);
+    const float Mn_use = (Mn == -INFINITY) ? 0.f : Mn;
+    // An empty sequence (M = -inf, num = den = 0) keeps a zero numerator.
+    f.fs = (M == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(M - Mn_use);
+    f.den = den * f.fs + __builtin_amdgcn_exp2f(z2 - Mn_use);
+    f.ref = Mn_use;
+  } else {
+    f.den += z;  // linear fold relative to the running max (flash_decode_cuda.cu:151-153)
+  }
+  return f;
 }
 
 // ---------------------------------------------------------------------------
@@ -1565,22 +1594,9 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) 
   float den = s_l[row][0];
 #pragma unroll
   for (int q = 1; q < kGroups; ++q) den += s_l[row][q];
-  float fs = 1.f;     // scale of the numerator for an exp sink
-  float ref = M_use;  // reference point of den
-  if (p.s_aux) {
-    if (p.sink_mode == FSK_SINK_EXP) {
-      // Extra logit z with a zero value vector (log2 domain: z * log2 e).
-      const float z2 = z * kLog2e;
-      const float Mn = fmaxf(M, z2);
-      const float Mn_use = (Mn == -INFINITY) ? 0.f : Mn;
-      // An empty sequence (M = -inf, num = den = 0) keeps a zero numerator.
-      fs = (M == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(M - Mn_use);
-      den = den * fs + __builtin_amdgcn_exp2f(z2 - Mn_use);
-      ref = Mn_use;
-    } else {
-      den += z;  // linear fold relative to the running max (flash_decode_cuda.cu:151-153)
-    }
-  }
+  const SinkFold sf = fold_sink(M, den, p.s_aux != nullptr, p.sink_mode, z);
+  den = sf.den;
+  const float ref = sf.ref;
 
   if (scores) {
     const int nvalid = (len_b + kScoreBlock - 1) / kScoreBlock;
@@ -1604,7 +1620,7 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) 
   f32x4 num = s_acc[row][0][d4];
 #pragma unroll
   for (int q = 1; q < kGroups; ++q) num += s_acc[row][q][d4];
-  if (p.s_aux && p.sink_mode == FSK_SINK_EXP) num *= fs;
+  if (p.s_aux && p.sink_mode == FSK_SINK_EXP) num *= sf.fs;
 
   uint8_t* o = p.out + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh;
   const f32x4 val = num / den;
@@ -1616,6 +1632,289 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) 
   } else {
     *(uint32_t __attribute__((ext_vector_type(2)))*)((bf16*)o + 4 * d4) =
         u32x2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Direct kernel: a short sequence's whole decode in one workgroup
+// ---------------------------------------------------------------------------
+// One workgroup of 1-8 waves per (sequence, head block): wave w takes tiles
+// w, w + W, ... of the sequence, on the partial kernel's tiles and pipeline,
+// and the waves' (m, l, acc) are merged through LDS, the sink folded and the
+// output (and block scores) stored.  No work plan, no partials in memory and
+// no second launch, which are most of a short call: what bounds it is the
+// chain kernel arguments -> lengths, page window and Q (one round trip: which
+// entries a wave needs does not depend on the length) -> tiles -> LDS merge.
+// The host takes it where the longest sequence the call can hold is short
+// enough for one workgroup (direct_waves has the rule and its figures).
+constexpr int kDirectMaxWaves = 8;
+constexpr int kDirectTokens = 1024;  // longest sequence extent of a direct call
+static_assert(kDirectTokens / 16 <= kWave, "one wave's page window holds every half tile");
+struct DirectParams {
+  Params p;
+  const float* s_aux;
+  int sink_mode;
+  uint8_t* out;
+  int64_t o_sb, o_sh;  // bytes
+  int o_dt;
+  int Hq;
+  uint8_t* scores;     // block scores [B, Hq, nblk] in the output dtype, or null
+  FastDiv last_cols;   // divisor: query heads of the last head block (with pair: of both KV heads)
+  int tiles;           // most tiles a sequence of the call can have (LDS of the block scores)
+  int host_lens;       // lengths below instead of the device's
+  int32_t start[kHostPlanMax], len[kHostPlanMax];
+};
+
+// LDS bytes of a wave: its K stage, then (aliased) its output sums (16 columns of D).
+template <int D, int kKV>
+constexpr int direct_region() {
+  using TR = TileRegs<D, kKV>;
+  constexpr int stage = (D <= 128 ? FSK_PIPE_DEPTH : 1) * 2 * TR::kHalfBytes;
+  return stage > 16 * D * 4 ? stage : 16 * D * 4;
+}
+// ... of a workgroup: the waves' regions, their m and l [16] and, with block
+// scores, every tile's maxima [16].
+template <int D, int kKV>
+constexpr uint32_t direct_lds(int waves, int score_tiles) {
+  return (uint32_t)(waves * (direct_region<D, kKV>() + 128) + score_tiles * 64);
+}
+
+template <int D, int kQ, int kKV, int kLayout>
+__global__ __launch_bounds__(kDirectMaxWaves * kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)))
+void direct_kernel(const int32_t* lens_arg, const int32_t* starts_arg, int B_arg, DirectParams dp) {
+  // (lengths first in the argument list: preloaded, as in the partial kernel)
+  Params p = dp.p;
+  p.lens = lens_arg;
+  p.starts = starts_arg;
+  p.B = B_arg;
+  using TR = TileRegs<D, kKV>;
+  using SM = Softmax<D, kQ, kKV>;
+  constexpr bool kKvFp8 = TR::kFp8;
+  constexpr int kSteps = SM::kSteps;
+  constexpr int kDpc = SM::kDpc;
+  constexpr int kDepth = (D <= 128) ? FSK_PIPE_DEPTH : 1;
+  constexpr int kRegion = direct_region<D, kKV>();
+
+  extern __shared__ __attribute__((aligned(16))) uint8_t s_direct[];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = uniform((int)threadIdx.x / kWave);
+  const int W = (int)blockDim.x / kWave;
+  const int g = lane >> 4;
+  const int c = lane & 15;
+  float* s_m = (float*)(s_direct + W * kRegion);  // [W][16]
+  float* s_l = s_m + W * 16;                      // [W][16]
+  float* s_tmax = s_l + W * 16;                   // [tiles][16] (block scores)
+  const uint32_t kstage = (uint32_t)(uintptr_t)s_direct + wave * kRegion;
+
+  const int b = blockIdx.y;
+  const int hh = blockIdx.x;
+  int start, len;
+  if (dp.host_lens) {
+    start = dp.start[b];
+    len = dp.len[b];
+  } else {
+    seq_range<kLayout>(p, b, start, len);
+  }
+  const int kvh0 = (int)fdiv((uint32_t)hh, p.hb_div);  // (with pair: the pair index, n_hb = 1)
+  const int hb = hh - kvh0 * p.n_hb;
+  const bool pair = (kLayout == kVarlen && D == 128) ? (uniform(p.pair) != 0) : false;
+  const int kvh = pair ? 2 * kvh0 : kvh0;
+
+  // Page ids of the wave's half tiles: half tile h2 of its k-th tile, token
+  // 32 (wave + k W) + 16 h2, in lane 2 k + h2 (a wave has at most 64).  Entries
+  // past the sequence are read (the table's row holds max_blocks of them,
+  // further ones read as 0) but not used.
+  int win = 0;
+  if constexpr (kLayout == kPaged) {
+    const auto rw = make_rsrc(p.block_table + (int64_t)b * p.bt_sb, 4 * p.max_blocks);
+    const uint32_t t = 32 * (wave + (lane >> 1) * W) + 16 * (lane & 1);
+    win = (int)buf_load<4>(rw, (int)(4 * fdiv(t, p.page))).w[0];
+  }
+
+  // Q^T operand, as in the partial kernel.
+  const int hs = (pair && c >= p.G) ? 1 : 0;
+  const int head = hb * 16 + c - hs * p.G;
+  const bool head_ok = head < p.G;
+  u32x4 qop[kSteps];
+  {
+    const uint8_t* qrow = p.q + (int64_t)b * p.q_sb + (int64_t)((kvh + hs) * p.G + (head_ok ? head : 0)) * p.q_sh;
+#pragma unroll
+    for (int i = 0; i < kSteps; ++i) {
+      const int dk = qk_dim0<kKvFp8>(i, g);
+      const int d0 = pair ? (dk & 63) : dk;
+      const bool q_ok = head_ok && (!pair || (dk >> 6) == hs);
+      u32x4 x;
+      if constexpr (kQ == kE4M3) {
+        const u32x2 raw = *(const u32x2*)(qrow + d0);
+        const float sq = p.q_scale[0];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(raw[e], false);
+          const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8(raw[e], true);
+          x[2 * e] = pack_f16x2(lo[0] * sq, lo[1] * sq);
+          x[2 * e + 1] = pack_f16x2(hi[0] * sq, hi[1] * sq);
+        }
+      } else {
+        x = *(const u32x4*)(qrow + 2 * d0);
+      }
+      qop[i] = q_ok ? x : u32x4{0, 0, 0, 0};
+    }
+  }
+  const float k_scale = kKvFp8 ? p.k_scale[0] : 1.0f;
+  const float v_scale = kKvFp8 ? p.v_scale[0] : 1.0f;
+  const LaneGeo<D, kKV> lg = lane_geo<D, kKV>(p, lane, g, c);
+  const float sscale = p.score_scale * k_scale;
+  if constexpr (kLayout == kPaged) win = clampi(win, 0, p.num_pages - 1);
+
+  start = uniform(start);
+  len = uniform(len);
+  const int n_all = (len + 31) >> 5;
+  const int n_tiles = n_all > wave ? (n_all - wave + W - 1) / W : 0;  // this wave's
+  auto half = [&](int k, int h2) {
+    HalfTile h;
+    const int t = 32 * (wave + k * W) + 16 * h2;
+    h.rows = uniform(clampi(len - t, 0, 16));
+    if constexpr (kLayout == kPaged) {
+      const int lp = (int)fdiv((uint32_t)t, p.page);
+      const int off = t - lp * p.page_size;
+      const int page = __builtin_amdgcn_readlane(win, (2 * k + h2) & 63);  // (< 64 while rows > 0)
+      h.k = p.k + (int64_t)page * p.k_s0 + kvh * p.k_sh + off * p.k_st;
+      h.v = p.v + (int64_t)page * p.v_s0 + kvh * p.v_sh + off * p.v_st;
+    } else {
+      const int64_t row = h.rows > 0 ? (int64_t)start + t : 0;
+      h.k = p.k + (kLayout == kDense ? (int64_t)b * p.k_s0 : 0) + kvh * p.k_sh + row * p.k_st;
+      h.v = p.v + (kLayout == kDense ? (int64_t)b * p.v_s0 : 0) + kvh * p.v_sh + row * p.v_st;
+    }
+    return h;
+  };
+  auto issue = [&](TR& T, int slot, int k) {
+    issue_tile<D, kKV>(T, kstage + slot * 2 * TR::kHalfBytes, p, [&](int h2) { return half(k, h2); }, lg);
+  };
+
+  SM st;
+  st.m_run = -INFINITY;
+  st.l_run = 0.f;
+#pragma unroll
+  for (int j = 0; j < kDpc; ++j) st.acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (n_tiles > 0) {
+    // (tiles past the wave's last one are issued with empty ranges, as in the
+    // partial kernel, so every wait has the same number of loads behind it)
+    TR tiles[kDepth];
+#pragma unroll
+    for (int q = 0; q < kDepth - 1; ++q) issue(tiles[q], q, q);
+    int k = 0;
+    bool done = false;
+    while (!done) {
+#pragma unroll
+      for (int q = 0; q < kDepth; ++q) {
+        if (!done) {
+          const int qn = (q + kDepth - 1) % kDepth;
+          issue(tiles[qn], qn, k + kDepth - 1);
+          wait_k_stage<TR::kLoads, kDepth>(kDepth - 1);
+          const float mt = compute_tile<D, kQ, kKV>(tiles[q], kstage + q * 2 * TR::kHalfBytes, st, qop, sscale, g, lg);
+          if (dp.scores && g == 0) s_tmax[(wave + k * W) * 16 + c] = mt;
+          ++k;
+          done = k >= n_tiles;
+        }
+      }
+    }
+  }
+  // The stage becomes the wave's output sums: the DMA loads of the empty
+  // tiles behind the last one have to have landed.
+  __builtin_amdgcn_s_waitcnt(vm_wait_imm(0));
+  asm volatile("" ::: "memory");
+  const float l_tot = group4_sum(st.l_run);
+  // Output sums as 16-byte pieces in lane order: piece i = r kDpc / 4 + j / 4
+  // of lane (g, c) holds dims kDpc (4 g + r) + j .. j + 3 of column c.  Writes
+  // and reads are free of bank conflicts ([column][dim] rows put 16 columns on
+  // the same banks: 16 query heads of 256 dims merged 3 us slower).
+  f32x4* s_acc = (f32x4*)(s_direct + wave * kRegion);  // [kDpc][64]
+  if (head_ok) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < kDpc; j += 4)
+        s_acc[(r * (kDpc / 4) + j / 4) * kWave + lane] =
+            f32x4{st.acc[j][r] * v_scale, st.acc[j + 1][r] * v_scale, st.acc[j + 2][r] * v_scale,
+                  st.acc[j + 3][r] * v_scale};
+  }
+  if (g == 0) {
+    s_m[wave * 16 + c] = st.m_run;
+    s_l[wave * 16 + c] = l_tot;
+  }
+  __syncthreads();
+
+  // ---- merge: a thread keeps one column, whose waves' weights it works out
+  // once, and takes pieces (piece * 4 + k-group) of it; with pair a column
+  // keeps its head's half of the k-groups
+  const int cols = pair ? 2 * p.G : min(16, p.G - hb * 16);
+  const FastDiv cols_div = hb == p.n_hb - 1 || pair ? dp.last_cols : FastDiv{16, 1, 4};
+  const int oe = dp.o_dt == FSK_F32 ? 4 : 2;
+  // Weights exp2(m_w - M) of a column's waves, its maximum and denominator.
+  struct Row {
+    float M, den, f[kDirectMaxWaves];
+  };
+  auto row_stats = [&](int col) {
+    Row R;
+    float m[kDirectMaxWaves];
+#pragma unroll
+    for (int w = 0; w < kDirectMaxWaves; ++w) m[w] = w < W ? s_m[w * 16 + col] : -INFINITY;
+    R.M = m[0];
+#pragma unroll
+    for (int w = 1; w < kDirectMaxWaves; ++w) R.M = fmaxf(R.M, m[w]);
+    const float mu = (R.M == -INFINITY) ? 0.f : R.M;
+    R.den = 0.f;
+#pragma unroll
+    for (int w = 0; w < kDirectMaxWaves; ++w) {
+      R.f[w] = __builtin_amdgcn_exp2f(m[w] - mu);
+      if (w < W) R.den += s_l[w * 16 + col] * R.f[w];
+    }
+    return R;
+  };
+  auto sink_of = [&](int oh, const Row& R) {
+    return fold_sink(R.M, R.den, dp.s_aux != nullptr, dp.sink_mode, dp.s_aux ? dp.s_aux[oh] : 0.f);
+  };
+  const int step = (int)fdiv(blockDim.x, cols_div);  // threads of a column (>= 4)
+  const int first = (int)fdiv(threadIdx.x, cols_div);
+  const int col = (int)threadIdx.x - first * cols;
+  const int hsel = (pair && col >= p.G) ? 1 : 0;
+  const int oh = (kvh + hsel) * p.G + (pair ? col - hsel * p.G : hb * 16 + col);
+  if (first < step) {
+    const Row R = row_stats(col);
+    const SinkFold sf = sink_of(oh, R);
+    uint8_t* orow = dp.out + (int64_t)b * dp.o_sb + (int64_t)oh * dp.o_sh;
+    for (int gi = first; gi < 4 * kDpc; gi += step) {
+      const int piece = gi >> 2, gg = gi & 3;
+      if (pair && (gg >> 1) != hsel) continue;
+      f32x4 num = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kDirectMaxWaves; ++w)
+        if (w < W) num += ((const f32x4*)(s_direct + w * kRegion))[piece * kWave + 16 * gg + col] * R.f[w];
+      if (dp.s_aux && dp.sink_mode == FSK_SINK_EXP) num *= sf.fs;
+      const f32x4 val = num / sf.den;
+      const int d = kDpc * 4 * gg + 4 * piece - hsel * 64;  // (piece = r kDpc / 4 + j / 4)
+      uint8_t* o = orow + d * oe;
+      if (dp.o_dt == FSK_F32) *(f32x4*)o = val;
+      else if (dp.o_dt == FSK_F16) *(u32x2*)o = u32x2{pack_f16x2(val[0], val[1]), pack_f16x2(val[2], val[3])};
+      else *(u32x2*)o = u32x2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
+    }
+  }
+  if (dp.scores && first < step) {
+    // largest probability of each block of four tiles; 0 past the sequence
+    const SinkFold sf = sink_of(oh, row_stats(col));
+    const float inv = 1.f / sf.den;
+    uint8_t* srow = dp.scores + ((int64_t)b * dp.Hq + oh) * p.nblk * oe;
+    for (int blk = first; blk < p.nblk; blk += step) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int q = 4 * blk; q < 4 * blk + 4; ++q)
+        if (q < n_all) mx = fmaxf(mx, s_tmax[q * 16 + col]);
+      const float sc = 4 * blk < n_all ? __builtin_amdgcn_exp2f(mx - sf.ref) * inv : 0.f;
+      uint8_t* dst = srow + blk * oe;
+      if (dp.o_dt == FSK_F32) *(float*)dst = sc;
+      else if (dp.o_dt == FSK_F16) *(f16*)dst = (f16)sc;
+      else *(bf16*)dst = (bf16)sc;
+    }
   }
 }
 
@@ -2232,6 +2531,7 @@ struct Options {
   int qk_engine = 0;            // 0: QK and PV on the matrix cores; 1: the VALU tile (A/B measurement)
   int head_pairs = 1;           // varlen, head_dim 64: neighbouring KV heads as one 128-wide row (see pair_shape)
   int seg_tokens = 96;          // lead-in per sequence in the work stream where boundaries are common (tokens)
+  int direct = 1;               // calls of short sequences on the direct kernel (see direct_waves); 0: never
 } g_opt;
 
 // Event triples of timed decode calls (the partial kernel's start and end and
@@ -2691,6 +2991,72 @@ int make_host_plan(const Common& c, const Params& p, HostPlan& hp) {
   return FSK_OK;
 }
 
+// The direct kernel's launch (see direct_waves).
+template <int D, int kQ, int kKV, int kLayout>
+void launch_direct(const DirectParams& dp, int waves, const Launch& s) {
+  const uint32_t lds = direct_lds<D, kKV>(waves, dp.scores ? dp.tiles : 0);
+  launch(direct_kernel<D, kQ, kKV, kLayout>, dim3((unsigned)dp.p.n_items_h, (unsigned)dp.p.B), dim3(waves * kWave), lds,
+         s, dp.p.lens, dp.p.starts, dp.p.B, dp);
+}
+template <int D, int kLayout>
+int dispatch_direct(const DirectParams& dp, int waves, int q_dt, int kv_dt, const Launch& s) {
+  if (kv_dt == FSK_F16) launch_direct<D, kF16, kF16, kLayout>(dp, waves, s);
+  else if (kv_dt == FSK_BF16) launch_direct<D, kBF16, kBF16, kLayout>(dp, waves, s);
+  else if (q_dt == FSK_F16) launch_direct<D, kF16, kE4M3, kLayout>(dp, waves, s);
+  else if (q_dt == FSK_BF16) launch_direct<D, kBF16, kE4M3, kLayout>(dp, waves, s);
+  else if constexpr (kLayout == kDense) launch_direct<D, kE4M3, kE4M3, kLayout>(dp, waves, s);
+  else return fail(FSK_ERR_UNSUPPORTED, "e4m3 q only on the dense layout");
+  return FSK_OK;
+}
+template <int D>
+int dispatch_direct_layout(int layout, const DirectParams& dp, int waves, int q_dt, int kv_dt, const Launch& s) {
+  if (layout == FSK_LAYOUT_VARLEN) return dispatch_direct<D, kVarlen>(dp, waves, q_dt, kv_dt, s);
+  if (layout == FSK_LAYOUT_PAGED) return dispatch_direct<D, kPaged>(dp, waves, q_dt, kv_dt, s);
+  return dispatch_direct<D, kDense>(dp, waves, q_dt, kv_dt, s);
+}
+
+// Waves of a direct call's workgroups, or 0: the split kernels.  `groups`
+// workgroups, one per (sequence, head slot).
+//
+// A workgroup streams from one CU at ~57 GB/s of fp16 K/V (2 MB in 37 us, by 4
+// waves or 8), the split kernels from all of them after ~5 us more of plan,
+// partials and second launch.  The line is drawn on the longest sequence the
+// call can hold (the table's or cache's width; varlen: all rows), since the
+// lengths are on the device: 192 KB of a head's K/V and 768 tokens for any
+// call, 512 KB and 1024 tokens where at least 128 workgroups spread over the
+// CUs.  16-bit rows of head_dim 256, whose tiles are not pipelined, stop at
+// 64 KB and 384 KB.  Paged, 8 KV heads x 128, us a step, split -> direct: fp16
+// 1 x 64 tokens 10.2 -> 6.9 (host time), 1 x 384 9.3 -> 7.4, 64 x 256 17.9 ->
+// 13.7, 256 x 64 23.8 -> 14.1, 256 x 512 94.7 -> 83.8, 1024 x U[1,256] 131 ->
+// 91, 16 x 1024 17.4 -> 15.3, 256 x U[1,1024] 100.9 -> 90.4; past the lines 4 x
+// 512 9.5 -> 9.0 (4 KV heads of 16 query heads: 9.7 -> 9.9), 4 x 1024 10.5 ->
+// 13.1, 64 x U[1,2048] 51.6 -> 53.0.  e4m3: 1 x 768 9.6 -> 9.0, 16 x 1024 13.4
+// -> 11.3, 256 x U[1,1024] 59.1 -> 51.5; past them 4 x 1024 10.1 -> 10.6, 4 x
+// 2048 11.9 -> 15.7.  fp16 head_dim 256: 1 x 64 10.1 -> 7.1, 64 x 384 39.9 ->
+// 34.3; past them 4 x 256 11.3 -> 12.0, 16 x 512 19.4 -> 20.0.
+//
+// Waves: one per two tiles, up to 8 in a few workgroups (1 x 512: 8.1 us with 4
+// waves, 7.8 with 8; 16 x 1024 e4m3 11.8 and 11.2) and 4 in many (64 x 512
+// fp16: 23.4 with 4, 26.1 with 8: fewer workgroups of 8 waves' stages fit a
+// CU); one per four tiles past 1024 workgroups (1024 x U[1,256]: 91.0 with 2,
+// 105.3 with 4; 1024 x 64: 48.6 with 1, 52.6 with 2).
+int direct_waves(const Common& c, int64_t groups) {
+  if (!g_opt.direct || c.chunk > 0 || g_opt.chunk_tokens > 0 || g_opt.qk_engine != 0) return 0;
+  const int64_t extent = c.layout == FSK_LAYOUT_PAGED ? c.kv_extent * c.page_size : c.kv_extent;
+  const int64_t row = 2 * (int64_t)c.D * elem_bytes(c.kv_dt);  // K/V bytes of a token and head
+  const bool many = groups >= 128;
+  const int64_t most_kb = c.D == 256 && c.kv_dt != FSK_E4M3 ? (many ? 384 : 64) : (many ? 512 : 192);
+  if (extent > (many ? kDirectTokens : 768) || extent * row > most_kb * 1024) return 0;
+  const int64_t tiles = cdiv(extent, 32);
+  const int64_t most = groups <= (c.kv_dt == FSK_E4M3 ? 128 : 16) ? kDirectMaxWaves : 4;
+  int waves = 1;
+  if (groups > 1024)
+    while (2 * waves <= std::min(tiles / 4, most)) waves *= 2;
+  else
+    while (waves < std::min(tiles <= 2 ? tiles : cdiv(tiles, 2), most)) waves *= 2;
+  return waves;
+}
+
 int run_decode(const Common& c) {
   int st = validate(c);
   if (st != FSK_OK) return st;
@@ -2765,6 +3131,37 @@ int run_decode(const Common& c) {
     st = make_host_plan(c, p, hp);
     if (st != FSK_OK) return st;
     p.lens = nullptr;  // (host memory: the kernel takes the plan instead)
+  }
+
+  if (const int waves = direct_waves(c, (int64_t)c.B * p.n_items_h)) {
+    DirectParams dp;
+    memset(&dp, 0, sizeof(dp));
+    dp.p = p;
+    dp.s_aux = c.s_aux; dp.sink_mode = c.sink_mode;
+    dp.out = (uint8_t*)c.out; dp.o_sb = c.o_sb * oe; dp.o_sh = c.o_sh * oe; dp.o_dt = c.o_dt;
+    dp.Hq = c.Hq;
+    dp.scores = (uint8_t*)c.scores;
+    dp.last_cols = make_fastdiv((uint32_t)(pair ? 2 * G : G - 16 * (n_hb - 1)));
+    dp.tiles = (int)cdiv(c.layout == FSK_LAYOUT_PAGED ? c.kv_extent * c.page_size : c.kv_extent, 32);
+    if (c.lens_on_host) {
+      dp.host_lens = 1;
+      memcpy(dp.start, hp.start, sizeof(dp.start));
+      memcpy(dp.len, hp.len, sizeof(dp.len));
+    }
+    (void)hipGetLastError();
+    // Timed calls: the dispatch stamps the kernel's start and end (the third
+    // event, recorded after it, keeps the record in triples).
+    hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+    if (!c.no_timing) timing_events(ev);
+    const Launch ld{c.stream, ev[0], ev[1]};
+    const int rc = c.D == 64 && !pair ? dispatch_direct_layout<64>(c.layout, dp, waves, c.q_dt, c.kv_dt, ld)
+                   : c.D <= 128       ? dispatch_direct_layout<128>(c.layout, dp, waves, c.q_dt, c.kv_dt, ld)
+                                      : dispatch_direct_layout<256>(c.layout, dp, waves, c.q_dt, c.kv_dt, ld);
+    timing_keep(ev, rc == FSK_OK && (!ev[0] || hipEventRecord(ev[2], c.stream) == hipSuccess));
+    if (rc != FSK_OK) return rc;
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(FSK_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(e));
+    return FSK_OK;
   }
 
   // Workgroups that can find a work item: no more than the workspace holds,
@@ -3024,6 +3421,11 @@ int fsk_set_option(const char* name, int64_t value) {
   if (!strcmp(name, "head_pairs")) {
     if (value != 0 && value != 1) return fail(FSK_ERR_INVALID, "head_pairs is 0 or 1");
     g_opt.head_pairs = (int)value;
+    return FSK_OK;
+  }
+  if (!strcmp(name, "direct")) {
+    if (value != 0 && value != 1) return fail(FSK_ERR_INVALID, "direct is 0 or 1");
+    g_opt.direct = (int)value;
     return FSK_OK;
   }
   if (!strcmp(name, "qk_engine")) {

@@ -394,6 +394,13 @@ FSK_API int fsk_quantize_e4m3(int count, const void *const *src, const int64_t *
  *   "head_pairs"          1 (default): varlen decodes at head_dim 64 with
  *                         packed heads read KV heads 2i and 2i+1 as one
  *                         128-wide row; 0: one KV head per wave
+ *   "direct"              1 (default): calls whose sequences are bounded to
+ *                         1024 tokens and 512 KB of a head's K/V (768 tokens
+ *                         and 192 KB with fewer than 128 workgroups; less for
+ *                         16-bit KV at head_dim 256) run one workgroup per
+ *                         sequence and head, with no partials and no reduce
+ *                         kernel; 0: always the split kernels.  (A fixed
+ *                         chunk_tokens split always takes the split kernels.)
  *   "qk_engine"           0 (default): QK and PV on the matrix cores (MFMA);
  *                         1: the VALU formulation of the tile, for A/B
  *                         measurement (f16 q and KV, head_dim 128, at most 4

@@ -99,6 +99,10 @@ constexpr float E4M3_MAX_F = 448.f;  // largest finite e4m3fn value
 
 enum Layout { kVarlen = 0, kPaged = 1, kDense = 2 };
 enum Kind { kF16 = FSK_F16, kBF16 = FSK_BF16, kF32 = FSK_F32, kE4M3 = FSK_E4M3 };
+// Q, K and V read as 16-bit values and quantised to e4m3 on the way to the
+// matrix cores (the HF attention function's fp8 form): kQuant + the type.
+constexpr int kQuant = 16;
+constexpr bool is_quant(int kind) { return kind >= kQuant; }
 
 __device__ __forceinline__ uint32_t f2u(float x) { return __builtin_bit_cast(uint32_t, x); }
 __device__ __forceinline__ float u2f(uint32_t x) { return __builtin_bit_cast(float, x); }
@@ -169,6 +173,103 @@ __device__ __forceinline__ f32x4 mfma16x16x32(u32x4 a, u32x4 b, f32x4 c) {
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+}
+
+// x / s rounded to fp32, for fp32 x and a scale s (finite, nonzero), from
+// rs = RN64(1 / s) as RN32(RN64(x * rs)).  This equals the correctly rounded
+// fp32 quotient: with x = X 2^a and s = S 2^b (X, S odd, < 2^24) the exact
+// quotient is never an fp32 rounding midpoint (a midpoint has 25 significant
+// bits, so m s = x would need an odd factor >= 2^24 + 1 in X) and lies at a
+// relative distance >= 1 / (2 S 2^24) >= 2^-49 from every midpoint, while the
+// two binary64 roundings perturb it by at most 2^-52 (1 + 2^-53) relative.
+// Quotients in the fp32 subnormal range may differ, but they all quantise to
+// a signed zero below.  Costs a convert, a multiply and a convert instead of
+// the ten-instruction fp32 division sequence.
+__device__ __forceinline__ float div_by_scale(float x, double rs) {
+  return (float)((double)x * rs);
+}
+
+// Four fp32 values -> four e4m3fn codes (round to nearest even, as torch's
+// float8_e4m3fn cast).  With a scale the values are first divided by it
+// (rs = 1 / scale in binary64, see div_by_scale) and clamped to +-448 (the
+// quantiser of fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16); without one
+// they are cast as they are, so magnitudes above 464 encode NaN as the cast
+// does.  NaN inputs are left to nan_codes.
+template <bool kScaled>
+__device__ __forceinline__ uint32_t encode_e4m3x4(const float* x, double rs) {
+  float y[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    y[j] = x[j];
+    if constexpr (kScaled) y[j] = fminf(fmaxf(div_by_scale(x[j], rs), -E4M3_MAX_F), E4M3_MAX_F);
+  }
+  int w = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], w, true);
+  return (uint32_t)w;
+}
+
+// NaN inputs take 0x7F with the input's sign bit, as torch's cast gives them.
+__device__ __forceinline__ uint32_t nan_codes(uint32_t u, const float* x) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (x[j] != x[j]) {
+      const uint32_t code = 0x7Fu | ((f2u(x[j]) >> 31) << 7);
+      u = (u & ~(0xFFu << (8 * j))) | (code << (8 * j));
+    }
+  }
+  return u;
+}
+
+// Four values -> four codes where the scale is infinite or NaN (the source
+// holds an infinity or a NaN): the fp32 quotient itself, NaNs by their sign.
+__device__ __forceinline__ uint32_t encode_e4m3x4_div(const float* x, float s) {
+  float y[4], z[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    y[j] = x[j] / s;
+    z[j] = fminf(fmaxf(y[j], -E4M3_MAX_F), E4M3_MAX_F);
+  }
+  return nan_codes(encode_e4m3x4<false>(z, 1.0), y);
+}
+
+// The per-tensor scale of a tensor whose |x| maximum has fp32 bits m
+// (fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16, as torch computes it):
+// clamp(min=1e-12) keeps NaN, and the division by the number 448 is torch's
+// multiplication by its fp32 reciprocal.
+struct QuantScale {
+  float s;
+  double rs;   // 1 / s
+  bool plain;  // m is finite, so s is a normal number
+};
+__device__ __forceinline__ QuantScale quant_scale(uint32_t m) {
+  QuantScale q;
+  const float amax = u2f(m);
+  q.s = (amax != amax ? amax : fmaxf(amax, 1e-12f)) * (1.0f / E4M3_MAX_F);
+  q.rs = 1.0 / (double)q.s;
+  q.plain = m < 0x7f800000u;
+  return q;
+}
+__device__ __forceinline__ uint32_t quant_codes4(const float* x, const QuantScale& q) {
+  return q.plain ? encode_e4m3x4<true>(x, q.rs) : encode_e4m3x4_div(x, q.s);
+}
+// Four 16-bit elements (two dwords) of type kSrc -> their codes, inside a
+// decode.  No clamp and no case apart: a tensor's own scale keeps every
+// quotient below 448 (1 + 2^-22), which rounds to 448, and where the scale is
+// infinite or NaN 1 / s is 0 or NaN, which gives the quotients 0 and NaN that
+// the division does (only a NaN code's sign may differ, and a decode does not
+// tell them apart).
+template <int kSrc>
+__device__ __forceinline__ uint32_t quant_codes4_of(uint32_t w0, uint32_t w1, const QuantScale& q) {
+  float x[4];
+  if constexpr (kSrc == kF16) {
+    const f16x2 a = __builtin_bit_cast(f16x2, w0), b = __builtin_bit_cast(f16x2, w1);
+    x[0] = (float)a[0]; x[1] = (float)a[1]; x[2] = (float)b[0]; x[3] = (float)b[1];
+  } else {
+    x[0] = bf16_lo_to_f32(w0); x[1] = bf16_hi_to_f32(w0); x[2] = bf16_lo_to_f32(w1); x[3] = bf16_hi_to_f32(w1);
+  }
+  int c = __builtin_amdgcn_cvt_pk_fp8_f32(div_by_scale(x[0], q.rs), div_by_scale(x[1], q.rs), 0, false);
+  c = __builtin_amdgcn_cvt_pk_fp8_f32(div_by_scale(x[2], q.rs), div_by_scale(x[3], q.rs), c, true);
+  return (uint32_t)c;
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, int bytes) {
@@ -273,6 +374,10 @@ struct Params {
   float* blk_max;
   int32_t* lens_out;
   int nblk;
+  // Quantising decode: |x| maxima of the workgroups that read Q, K and V
+  // (amax_n entries each, one tensor after the other).
+  const uint32_t* amax;
+  int amax_n[3];
 };
 
 // A plan built on the host (the host-plan entry points, for callers that
@@ -882,12 +987,75 @@ struct Softmax {
   f32x4 acc[kDpc];
 };
 
+// Scales of a quantising decode (empty otherwise).  Every wave works them out
+// from the partial maxima, which it loads before its plan.
+template <int kKV>
+struct Requant {};
+template <>
+struct Requant<kQuant + kF16> {
+  QuantScale q, k, v;
+};
+template <>
+struct Requant<kQuant + kBF16> {
+  QuantScale q, k, v;
+};
+constexpr int kAmaxMax = 256;  // partial maxima of a tensor at most
+template <int kKV>
+struct AmaxLoads {
+  uint32_t m[3][kAmaxMax / kWave];
+};
+template <int kKV>
+__device__ __forceinline__ void amax_issue(const Params& p, int lane, AmaxLoads<kKV>& a) {
+  if constexpr (is_quant(kKV)) {
+    const uint32_t* part = p.amax;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+      for (int i = 0; i < kAmaxMax / kWave; ++i) a.m[t][i] = part[min(lane + i * kWave, p.amax_n[t] - 1)];
+      part += p.amax_n[t];
+    }
+  }
+}
+template <int kKV>
+__device__ __forceinline__ void amax_scales(const AmaxLoads<kKV>& a, Requant<kKV>& rq) {
+  if constexpr (is_quant(kKV)) {
+    uint32_t m[3];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      m[t] = a.m[t][0];
+#pragma unroll
+      for (int i = 1; i < kAmaxMax / kWave; ++i) m[t] = max(m[t], a.m[t][i]);
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1)
+#pragma unroll
+      for (int t = 0; t < 3; ++t) m[t] = max(m[t], (uint32_t)__shfl_xor((int)m[t], o));
+    rq.q = quant_scale((uint32_t)uniform((int)m[0]));
+    rq.k = quant_scale((uint32_t)uniform((int)m[1]));
+    rq.v = quant_scale((uint32_t)uniform((int)m[2]));
+  }
+}
+// Eight 16-bit Q elements -> their codes' values times the scale, as f16 (q =
+// f16(f32(q8) * scale_q), triton_gqa_decode_hf_fp8.py:47-50).
+__device__ __forceinline__ u32x4 q_operand(u32x2 codes, float sq) {
+  u32x4 x;
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const uint32_t w = codes[e];
+    const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
+    const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8(w, true);
+    x[2 * e] = pack_f16x2(lo[0] * sq, lo[1] * sq);
+    x[2 * e + 1] = pack_f16x2(hi[0] * sq, hi[1] * sq);
+  }
+  return x;
+}
+
 // Returns the tile's maximum score of head column c (log2 domain, -inf when
 // the tile has no valid row).
 template <int D, int kQ, int kKV>
 __device__ __forceinline__ float compute_tile(const TileRegs<D, kKV>& T, uint32_t kstage,
                                               Softmax<D, kQ, kKV>& st, const u32x4 (&qop)[D / 32], float sscale,
-                                              int g, const LaneGeo<D, kKV>& lg) {
+                                              int g, const LaneGeo<D, kKV>& lg, const Requant<kKV>& rq) {
   using TR = TileRegs<D, kKV>;
   using SM = Softmax<D, kQ, kKV>;
   constexpr int kSteps = SM::kSteps;
@@ -906,6 +1074,11 @@ __device__ __forceinline__ float compute_tile(const TileRegs<D, kKV>& T, uint32_
         const u32x4 raw = *(lds_u32x4*)(uintptr_t)(kstage + h2 * TR::kHalfBytes + lg.kread[i >> 1]);
         const u32x2 a = e4m3x4_to<SM::kQkBf16>(raw[2 * (i & 1)]);
         const u32x2 bb = e4m3x4_to<SM::kQkBf16>(raw[2 * (i & 1) + 1]);
+        kop = u32x4{a[0], a[1], bb[0], bb[1]};
+      } else if constexpr (is_quant(kKV)) {
+        const u32x4 raw = *(lds_u32x4*)(uintptr_t)(kstage + h2 * TR::kHalfBytes + lg.kread[i]);
+        const u32x2 a = e4m3x4_to<false>(quant_codes4_of<kKV - kQuant>(raw[0], raw[1], rq.k));
+        const u32x2 bb = e4m3x4_to<false>(quant_codes4_of<kKV - kQuant>(raw[2], raw[3], rq.k));
         kop = u32x4{a[0], a[1], bb[0], bb[1]};
       } else {
         kop = *(lds_u32x4*)(uintptr_t)(kstage + h2 * TR::kHalfBytes + lg.kread[i]);
@@ -974,6 +1147,13 @@ __device__ __forceinline__ float compute_tile(const TileRegs<D, kKV>& T, uint32_
         const u32x2 x = e4m3x4_to<false>(T.v[sidx].w[e]);
         vw[sidx][2 * e] = x[0];
         vw[sidx][2 * e + 1] = x[1];
+      }
+    } else if constexpr (is_quant(kKV)) {
+#pragma unroll
+      for (int e = 0; e < kVWords; e += 2) {
+        const u32x2 x = e4m3x4_to<false>(quant_codes4_of<kKV - kQuant>(T.v[sidx].w[e], T.v[sidx].w[e + 1], rq.v));
+        vw[sidx][e] = x[0];
+        vw[sidx][e + 1] = x[1];
       }
     } else {
 #pragma unroll
@@ -1194,8 +1374,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
   const LaneGeo<D, kKV> lg = lane_geo<D, kKV>(p, lane, g, c);
   // The KV scales, read before the plan (their round trip overlaps the
   // lengths') and used after it.
-  const float k_scale = kKvFp8 ? p.k_scale[0] : 1.0f;
-  const float v_scale = kKvFp8 ? p.v_scale[0] : 1.0f;
+  float k_scale = kKvFp8 ? p.k_scale[0] : 1.0f;
+  float v_scale = kKvFp8 ? p.v_scale[0] : 1.0f;
+  AmaxLoads<kKV> am;
+  amax_issue<kKV>(p, lane, am);
   if constexpr (kHostPlan) {
     // Workgroup 0 publishes the unit prefix for the reduce kernel, as
     // build_plan does (lanes past B hold pre[B]).
@@ -1205,6 +1387,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
     }
   } else {
     sp = build_plan<kLayout, kScores>(p, s_pre, s_flat, lane_len, seg_x, lane_flat, lane_pre);
+  }
+  Requant<kKV> rq;
+  amax_scales<kKV>(am, rq);
+  if constexpr (is_quant(kKV)) {
+    k_scale = rq.k.s;
+    v_scale = rq.v.s;
   }
   FSK_STAMP(1);
   int segments_done = 0;
@@ -1289,16 +1477,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
         // unconditional loads keep the compiler's wait counts exact.
         u32x4 x;
         if constexpr (kQ == kE4M3) {
-          // q = f16(f32(q8) * scale_q)  (triton_gqa_decode_hf_fp8.py:47-50)
-          const u32x2 raw = *(const u32x2*)(qrow + d0);
-          const float sq = p.q_scale[0];
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(raw[e], false);
-            const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8(raw[e], true);
-            x[2 * e] = pack_f16x2(lo[0] * sq, lo[1] * sq);
-            x[2 * e + 1] = pack_f16x2(hi[0] * sq, hi[1] * sq);
-          }
+          x = q_operand(*(const u32x2*)(qrow + d0), p.q_scale[0]);
+        } else if constexpr (is_quant(kQ)) {
+          const u32x4 raw = *(const u32x4*)(qrow + 2 * d0);
+          x = q_operand(u32x2{quant_codes4_of<kQ - kQuant>(raw[0], raw[1], rq.q),
+                              quant_codes4_of<kQ - kQuant>(raw[2], raw[3], rq.q)}, rq.q.s);
         } else {
           x = *(const u32x4*)(qrow + 2 * d0);
         }
@@ -1379,7 +1562,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
               compute_tile_valu<D>(tiles[s], s_kstage + s * 2 * TR::kHalfBytes, sv, qv, sscale, g, c);
             } else {
               const float mt = compute_tile<D, kQ, kKV>(tiles[s], s_kstage + s * 2 * TR::kHalfBytes, st, qop,
-                                                        sscale, g, lg);
+                                                        sscale, g, lg, rq);
               if constexpr (kScores) bm.add(p, un, un.t_begin + 32 * k, mt, head, head_ok, g);
             }
             ++k;
@@ -1396,7 +1579,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
         if constexpr (kValu) {
           compute_tile_valu<D>(ta, s_kstage, sv, qv, sscale, g, c);
         } else {
-          const float mt = compute_tile<D, kQ, kKV>(ta, s_kstage, st, qop, sscale, g, lg);
+          const float mt = compute_tile<D, kQ, kKV>(ta, s_kstage, st, qop, sscale, g, lg, rq);
           if constexpr (kScores) bm.add(p, un, t, mt, head, head_ok, g);
         }
       }
@@ -1731,6 +1914,11 @@ void direct_kernel(const int32_t* lens_arg, const int32_t* starts_arg, int B_arg
     win = (int)buf_load<4>(rw, (int)(4 * fdiv(t, p.page))).w[0];
   }
 
+  AmaxLoads<kKV> am;
+  Requant<kKV> rq;
+  amax_issue<kKV>(p, lane, am);
+  amax_scales<kKV>(am, rq);
+
   // Q^T operand, as in the partial kernel.
   const int hs = (pair && c >= p.G) ? 1 : 0;
   const int head = hb * 16 + c - hs * p.G;
@@ -1745,23 +1933,23 @@ void direct_kernel(const int32_t* lens_arg, const int32_t* starts_arg, int B_arg
       const bool q_ok = head_ok && (!pair || (dk >> 6) == hs);
       u32x4 x;
       if constexpr (kQ == kE4M3) {
-        const u32x2 raw = *(const u32x2*)(qrow + d0);
-        const float sq = p.q_scale[0];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const f32x2 lo = __builtin_amdgcn_cvt_pk_f32_fp8(raw[e], false);
-          const f32x2 hi = __builtin_amdgcn_cvt_pk_f32_fp8(raw[e], true);
-          x[2 * e] = pack_f16x2(lo[0] * sq, lo[1] * sq);
-          x[2 * e + 1] = pack_f16x2(hi[0] * sq, hi[1] * sq);
-        }
+        x = q_operand(*(const u32x2*)(qrow + d0), p.q_scale[0]);
+      } else if constexpr (is_quant(kQ)) {
+        const u32x4 raw = *(const u32x4*)(qrow + 2 * d0);
+        x = q_operand(u32x2{quant_codes4_of<kQ - kQuant>(raw[0], raw[1], rq.q),
+                            quant_codes4_of<kQ - kQuant>(raw[2], raw[3], rq.q)}, rq.q.s);
       } else {
         x = *(const u32x4*)(qrow + 2 * d0);
       }
       qop[i] = q_ok ? x : u32x4{0, 0, 0, 0};
     }
   }
-  const float k_scale = kKvFp8 ? p.k_scale[0] : 1.0f;
-  const float v_scale = kKvFp8 ? p.v_scale[0] : 1.0f;
+  float k_scale = kKvFp8 ? p.k_scale[0] : 1.0f;
+  float v_scale = kKvFp8 ? p.v_scale[0] : 1.0f;
+  if constexpr (is_quant(kKV)) {
+    k_scale = rq.k.s;
+    v_scale = rq.v.s;
+  }
   const LaneGeo<D, kKV> lg = lane_geo<D, kKV>(p, lane, g, c);
   const float sscale = p.score_scale * k_scale;
   if constexpr (kLayout == kPaged) win = clampi(win, 0, p.num_pages - 1);
@@ -1811,7 +1999,7 @@ void direct_kernel(const int32_t* lens_arg, const int32_t* starts_arg, int B_arg
           const int qn = (q + kDepth - 1) % kDepth;
           issue(tiles[qn], qn, k + kDepth - 1);
           wait_k_stage<TR::kLoads, kDepth>(kDepth - 1);
-          const float mt = compute_tile<D, kQ, kKV>(tiles[q], kstage + q * 2 * TR::kHalfBytes, st, qop, sscale, g, lg);
+          const float mt = compute_tile<D, kQ, kKV>(tiles[q], kstage + q * 2 * TR::kHalfBytes, st, qop, sscale, g, lg, rq);
           if (dp.scores && g == 0) s_tmax[(wave + k * W) * 16 + c] = mt;
           ++k;
           done = k >= n_tiles;
@@ -2059,51 +2247,6 @@ __device__ __forceinline__ void widen8(const WriteRow& w, float (&x)[8]) {
   }
 }
 
-// x / s rounded to fp32, for fp32 x and a scale s (finite, nonzero), from
-// rs = RN64(1 / s) as RN32(RN64(x * rs)).  This equals the correctly rounded
-// fp32 quotient: with x = X 2^a and s = S 2^b (X, S odd, < 2^24) the exact
-// quotient is never an fp32 rounding midpoint (a midpoint has 25 significant
-// bits, so m s = x would need an odd factor >= 2^24 + 1 in X) and lies at a
-// relative distance >= 1 / (2 S 2^24) >= 2^-49 from every midpoint, while the
-// two binary64 roundings perturb it by at most 2^-52 (1 + 2^-53) relative.
-// Quotients in the fp32 subnormal range may differ, but they all quantise to
-// a signed zero below.  Costs a convert, a multiply and a convert instead of
-// the ten-instruction fp32 division sequence.
-__device__ __forceinline__ float div_by_scale(float x, double rs) {
-  return (float)((double)x * rs);
-}
-
-// Four fp32 values -> four e4m3fn codes (round to nearest even, as torch's
-// float8_e4m3fn cast).  With a scale the values are first divided by it
-// (rs = 1 / scale in binary64, see div_by_scale) and clamped to +-448 (the
-// quantiser of fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16); without one
-// they are cast as they are, so magnitudes above 464 encode NaN as the cast
-// does.  NaN inputs are left to nan_codes.
-template <bool kScaled>
-__device__ __forceinline__ uint32_t encode_e4m3x4(const float* x, double rs) {
-  float y[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    y[j] = x[j];
-    if constexpr (kScaled) y[j] = fminf(fmaxf(div_by_scale(x[j], rs), -E4M3_MAX_F), E4M3_MAX_F);
-  }
-  int w = __builtin_amdgcn_cvt_pk_fp8_f32(y[0], y[1], 0, false);
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(y[2], y[3], w, true);
-  return (uint32_t)w;
-}
-
-// NaN inputs take 0x7F with the input's sign bit, as torch's cast gives them.
-__device__ __forceinline__ uint32_t nan_codes(uint32_t u, const float* x) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (x[j] != x[j]) {
-      const uint32_t code = 0x7Fu | ((f2u(x[j]) >> 31) << 7);
-      u = (u & ~(0xFFu << (8 * j))) | (code << (8 * j));
-    }
-  }
-  return u;
-}
-
 template <int kPool>
 __device__ __forceinline__ uint32_t pack2(float a, float b) {
   if constexpr (kPool == kF16) return pack_f16x2(a, b);
@@ -2212,13 +2355,13 @@ __global__ __launch_bounds__(kWriteThreads) void kv_write_kernel(WriteParams p) 
 // ---------------------------------------------------------------------------
 // scale = max(max|x|, 1e-12) / 448, codes = e4m3(clamp(x / scale, +-448)), in
 // fp32 as torch computes them (16-bit sources are widened first).  Two
-// launches for up to three tensors (an attention call's Q, K and V): every
-// workgroup's |x| maximum, then the codes.  HBM-bound: the source is read
-// twice (the second time largely from the 256 MB Infinity Cache) and the codes
-// written once.  As torch operations this was eight passes over fp32 copies:
-// Q, K and V of 4 x 8 heads x 3827 tokens x 128 (bf16, 62.7 MB) in 24 launches,
-// 259 us; now the maxima take 13.2 us and the codes 17.1 us (traced), and the
-// fp8 attention call 45.6 us instead of 311 (with mask_bounds_kernel).
+// launches for up to three tensors: every workgroup's |x| maximum, then the
+// codes.  HBM-bound: the source is read twice (the second time largely from
+// the 256 MB Infinity Cache) and the codes written once.  As torch operations
+// this was eight passes over fp32 copies: Q, K and V of 4 x 8 heads x 3827
+// tokens x 128 (bf16, 62.7 MB) in 24 launches, 259 us; the maxima take 13 us
+// and the codes 17 us (traced).  The attention hook's fp8 form does not store
+// the codes at all (bounds_amax_kernel and the decode kernels' kQuant kinds).
 constexpr int kQuantMax = 3;         // tensors per call
 constexpr int kQuantThreads = 256;
 constexpr int kQuantStep = 16;       // elements of a thread's step: one 16-byte store of codes
@@ -2276,55 +2419,43 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t m) {
   return m;
 }
 
+// |x| maximum of the elements of workgroup `blk` (of t.nblk) of a tensor, for
+// every thread: four steps of loads in flight per thread.
 template <int kSrc>
-__global__ __launch_bounds__(kQuantThreads) void quant_amax_kernel(QuantParams p) {
+__device__ __forceinline__ uint32_t quant_amax_block(const QuantTensor& t, uint32_t blk) {
   constexpr int kE = kSrc == kF32 ? 4 : 2;   // bytes per element
   constexpr int kV = kQuantStep * kE / 16;   // 16-byte loads per step
-  const QuantTensor t = quant_tensor(p);
+  constexpr int kFlight = 4;
   const int64_t steps = t.n / kQuantStep;
   const int64_t stride = (int64_t)t.nblk * kQuantThreads;
-  int64_t i = (int64_t)(blockIdx.x - t.blk0) * kQuantThreads + threadIdx.x;
   uint32_t m = 0;
-  for (; i + stride < steps; i += 2 * stride) {  // two steps in flight
-    u32x4 x[2 * kV];
+  for (int64_t i = (int64_t)blk * kQuantThreads + threadIdx.x; i < steps; i += kFlight * stride) {
+    u32x4 x[kFlight * kV];
 #pragma unroll
-    for (int j = 0; j < kV; ++j) {
-      x[j] = ((const u32x4*)t.src)[i * kV + j];
-      x[kV + j] = ((const u32x4*)t.src)[(i + stride) * kV + j];
+    for (int f = 0; f < kFlight; ++f) {
+      const int64_t at = min(i + f * stride, steps - 1);  // (a repeated step changes nothing)
+#pragma unroll
+      for (int j = 0; j < kV; ++j) x[f * kV + j] = ((const u32x4*)t.src)[at * kV + j];
     }
 #pragma unroll
-    for (int j = 0; j < 2 * kV; ++j)
+    for (int j = 0; j < kFlight * kV; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e) m = abs_max<kSrc>(m, x[j][e]);
   }
-  if (i < steps) {
-#pragma unroll
-    for (int j = 0; j < kV; ++j) {
-      const u32x4 x = ((const u32x4*)t.src)[i * kV + j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) m = abs_max<kSrc>(m, x[e]);
-    }
-  }
   // the elements past the last whole step
   const int64_t tail = steps * kQuantStep + threadIdx.x;
-  if (blockIdx.x == t.blk0 && tail < t.n) {
+  if (blk == 0 && tail < t.n) {
     const uint32_t x = kE == 4 ? ((const uint32_t*)t.src)[tail] : (uint32_t)((const uint16_t*)t.src)[tail];
     m = abs_max<kSrc>(m, x);
   }
-  m = block_max_u32(abs_max_f32<kSrc>(m));
-  if (threadIdx.x == 0) p.part[blockIdx.x] = m;
+  return block_max_u32(abs_max_f32<kSrc>(m));
 }
 
-// Four values -> four codes where the scale is infinite or NaN (the source
-// holds an infinity or a NaN): the fp32 quotient itself, NaNs by their sign.
-__device__ __forceinline__ uint32_t encode_e4m3x4_div(const float* x, float s) {
-  float y[4], z[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    y[j] = x[j] / s;
-    z[j] = fminf(fmaxf(y[j], -E4M3_MAX_F), E4M3_MAX_F);
-  }
-  return nan_codes(encode_e4m3x4<false>(z, 1.0), y);
+template <int kSrc>
+__global__ __launch_bounds__(kQuantThreads) void quant_amax_kernel(QuantParams p) {
+  const QuantTensor t = quant_tensor(p);
+  const uint32_t m = quant_amax_block<kSrc>(t, blockIdx.x - t.blk0);
+  if (threadIdx.x == 0) p.part[blockIdx.x] = m;
 }
 
 template <int kSrc>
@@ -2352,14 +2483,9 @@ __global__ __launch_bounds__(kQuantThreads) void quant_codes_kernel(QuantParams 
   uint32_t m = 0;
   for (uint32_t j = threadIdx.x; j < t.nblk; j += kQuantThreads) m = max(m, p.part[t.blk0 + j]);
   m = block_max_u32(m);
-  const float amax = u2f(m);
-  // clamp(min=1e-12) keeps NaN; the division by the number 448 is torch's
-  // multiplication by its fp32 reciprocal
-  const float s = (amax != amax ? amax : fmaxf(amax, 1e-12f)) * (1.0f / E4M3_MAX_F);
-  if (blockIdx.x == t.blk0 && threadIdx.x == 0) *t.scale = s;
-  const bool plain = m < 0x7f800000u;  // finite: s is a normal number
-  const double rs = 1.0 / (double)s;
-  auto codes4 = [&](const float* x) { return plain ? encode_e4m3x4<true>(x, rs) : encode_e4m3x4_div(x, s); };
+  const QuantScale qs = quant_scale(m);
+  if (blockIdx.x == t.blk0 && threadIdx.x == 0) *t.scale = qs.s;
+  auto codes4 = [&](const float* x) { return quant_codes4(x, qs); };
   while (i < steps) {
     float x[kQuantStep];
 #pragma unroll
@@ -2412,7 +2538,9 @@ struct BoundsParams {
   int64_t m_sb, m_ss;       // batch / position strides, bytes
   const int64_t* position;  // without a mask: the step's position, or null (length S)
   int64_t window;           // without a mask: attend the last `window` positions (< 0: all)
+  int mask_kind;            // element type, or -1 without a mask
   int B, S;
+  int blocks;               // workgroups
   int32_t* ends;
   int32_t* starts;          // or null (without a mask and window)
 };
@@ -2444,11 +2572,10 @@ __device__ __forceinline__ bool attended(const uint8_t* p) {
 }
 
 template <int kM>
-__global__ __launch_bounds__(kBoundsThreads) void mask_bounds_kernel(BoundsParams p) {
+__device__ __forceinline__ void mask_bounds_block(const BoundsParams& p, int b) {
   constexpr int kSize = kM == kF32 ? 4 : kM == kBool ? 1 : 2;
   constexpr int kE = 16 / kSize;  // elements of a 16-byte load
   constexpr int kUnroll = 4;
-  const int b = blockIdx.x;
   const uint8_t* row = p.mask + b * p.m_sb;
   int first = p.S, end = 0;
   auto take = [&](int i) {
@@ -2503,13 +2630,47 @@ __global__ __launch_bounds__(kBoundsThreads) void mask_bounds_kernel(BoundsParam
   p.starts[b] = min(first, end);
 }
 
-// Without a mask: every sequence of the batch has the same range.
-__global__ __launch_bounds__(kBoundsThreads) void position_bounds_kernel(BoundsParams p) {
-  const int b = blockIdx.x * kBoundsThreads + threadIdx.x;
+// Without a mask every sequence of the batch has the same range; a workgroup
+// writes kBoundsThreads of them.
+__device__ __forceinline__ void position_bounds_block(const BoundsParams& p, int blk) {
+  const int b = blk * kBoundsThreads + threadIdx.x;
   if (b >= p.B) return;
   const int len = p.position ? (int)(*p.position + 1) : p.S;
   p.ends[b] = len;
   if (p.starts) p.starts[b] = (int)max((int64_t)len - p.window, (int64_t)0);
+}
+
+// mask_kind: a mask's element type, or -1 for none (workgroup-uniform).
+__device__ __forceinline__ void bounds_block(const BoundsParams& p, int blk) {
+  if (p.mask_kind < 0) position_bounds_block(p, blk);
+  else if (p.mask_kind == kBool) mask_bounds_block<kBool>(p, blk);
+  else if (p.mask_kind == kF32) mask_bounds_block<kF32>(p, blk);
+  else mask_bounds_block<kF16>(p, blk);  // (f16 and bf16 zeros alike)
+}
+__global__ __launch_bounds__(kBoundsThreads) void bounds_kernel(BoundsParams p) { bounds_block(p, blockIdx.x); }
+
+// The first launch of a quantising decode: the attended ranges (workgroups
+// [0, p.blocks)) and the |x| maxima of Q, K and V, which do not depend on each
+// other.  The decode kernels take the scales from the maxima and quantise the
+// 16-bit rows between LDS and the matrix cores, so the codes are neither
+// written nor read: 4 x 8 heads x 3827 tokens x 128 bf16, ranges + maxima 12.6
+// us and the partial kernel 16.6 (16-bit rows alone 15, codes 10), against 2.6 +
+// 13 + 17 + 10 us with stored codes; the call 45.6 -> 31.8 us, and 26.5 -> 11.4
+// for one of 50 tokens (two launches instead of four).  The conversion is not
+// what bounds it: an fp32 quotient of two FMAs instead of the binary64 one
+// measured the same 16.5 us, a branch around it for infinite scales 24 us (10K
+// instructions, with the clamp).
+template <int kSrc>
+__global__ __launch_bounds__(kQuantThreads) void bounds_amax_kernel(BoundsParams bp, QuantParams p) {
+  static_assert(kQuantThreads == kBoundsThreads, "one workgroup size");
+  if ((int)blockIdx.x < bp.blocks) {
+    bounds_block(bp, blockIdx.x);
+    return;
+  }
+  const uint32_t w = blockIdx.x - bp.blocks;
+  const QuantTensor t = w >= p.t[2].blk0 ? p.t[2] : w >= p.t[1].blk0 ? p.t[1] : p.t[0];
+  const uint32_t m = quant_amax_block<kSrc>(t, w - t.blk0);
+  if (threadIdx.x == 0) p.part[w] = m;
 }
 
 // ---------------------------------------------------------------------------
@@ -2732,6 +2893,7 @@ struct Common {
   hipStream_t stream;
   void* scores; int nblk;  // block scores [B, Hq, nblk] in the output dtype, or null
   bool no_timing;          // never stamp this call (no event creation: the allocation-free entry)
+  const struct QuantPre* pre;  // quantising decode (dense, f16 / bf16): its first launch, or null
   bool lens_on_host;       // lens is host memory: the plan is built here (make_host_plan)
 };
 
@@ -2829,6 +2991,13 @@ void launch_partial(const Params& p, int grid, const Launch& s) {
 
 template <int D, int kLayout, bool kScores>
 int dispatch_qkv(const Params& p, int grid, int q_dt, int kv_dt, const Launch& s) {
+  if constexpr (kLayout == kDense && !kScores) {
+    if (p.amax) {
+      if (kv_dt == FSK_F16) launch_partial<D, kQuant + kF16, kQuant + kF16, kLayout, kScores>(p, grid, s);
+      else launch_partial<D, kQuant + kBF16, kQuant + kBF16, kLayout, kScores>(p, grid, s);
+      return FSK_OK;
+    }
+  }
   if (kv_dt == FSK_F16) launch_partial<D, kF16, kF16, kLayout, kScores>(p, grid, s);
   else if (kv_dt == FSK_BF16) launch_partial<D, kBF16, kBF16, kLayout, kScores>(p, grid, s);
   else if (q_dt == FSK_F16) launch_partial<D, kF16, kE4M3, kLayout, kScores>(p, grid, s);
@@ -2991,6 +3160,19 @@ int make_host_plan(const Common& c, const Params& p, HostPlan& hp) {
   return FSK_OK;
 }
 
+// The first launch of a quantising decode (run_quant_decode).
+struct QuantPre {
+  BoundsParams bp;
+  QuantParams qp;
+  unsigned grid;
+  int dt;
+};
+void launch_pre(const QuantPre& q, hipStream_t stream) {
+  const Launch l{stream, nullptr, nullptr};
+  if (q.dt == FSK_F16) launch(bounds_amax_kernel<kF16>, dim3(q.grid), dim3(kQuantThreads), 0, l, q.bp, q.qp);
+  else launch(bounds_amax_kernel<kBF16>, dim3(q.grid), dim3(kQuantThreads), 0, l, q.bp, q.qp);
+}
+
 // The direct kernel's launch (see direct_waves).
 template <int D, int kQ, int kKV, int kLayout>
 void launch_direct(const DirectParams& dp, int waves, const Launch& s) {
@@ -3000,6 +3182,13 @@ void launch_direct(const DirectParams& dp, int waves, const Launch& s) {
 }
 template <int D, int kLayout>
 int dispatch_direct(const DirectParams& dp, int waves, int q_dt, int kv_dt, const Launch& s) {
+  if constexpr (kLayout == kDense) {
+    if (dp.p.amax) {
+      if (kv_dt == FSK_F16) launch_direct<D, kQuant + kF16, kQuant + kF16, kLayout>(dp, waves, s);
+      else launch_direct<D, kQuant + kBF16, kQuant + kBF16, kLayout>(dp, waves, s);
+      return FSK_OK;
+    }
+  }
   if (kv_dt == FSK_F16) launch_direct<D, kF16, kF16, kLayout>(dp, waves, s);
   else if (kv_dt == FSK_BF16) launch_direct<D, kBF16, kBF16, kLayout>(dp, waves, s);
   else if (q_dt == FSK_F16) launch_direct<D, kF16, kE4M3, kLayout>(dp, waves, s);
@@ -3101,6 +3290,10 @@ int run_decode(const Common& c) {
   p.nh_div = make_fastdiv((uint32_t)p.n_items_h);
   p.hb_div = make_fastdiv((uint32_t)p.n_hb);
   p.hkv_div = make_fastdiv((uint32_t)c.Hkv);
+  if (c.pre) {
+    p.amax = c.pre->qp.part;
+    for (int i = 0; i < 3; ++i) p.amax_n[i] = (int)c.pre->qp.t[i].nblk;
+  }
   // The skew is not applied to a fixed split, nor at head_dim 256: there the
   // even and odd XCDs stream at the same rate (16-bit KV: partial kernel
   // 3-4 % slower with it, paged and varlen; e4m3: no difference).
@@ -3133,6 +3326,7 @@ int run_decode(const Common& c) {
     p.lens = nullptr;  // (host memory: the kernel takes the plan instead)
   }
 
+  if (c.pre) launch_pre(*c.pre, c.stream);
   if (const int waves = direct_waves(c, (int64_t)c.B * p.n_items_h)) {
     DirectParams dp;
     memset(&dp, 0, sizeof(dp));
@@ -3356,16 +3550,16 @@ int run_quantize(int count, const void* const* src, const int64_t* numel, int sr
   return FSK_OK;
 }
 
-int run_bounds(const void* mask, int mask_dt, int64_t sb, int64_t ss, const int64_t* position, int64_t window, int B,
-               int S, int32_t* ends, int32_t* starts, hipStream_t stream) {
+int make_bounds(const void* mask, int mask_dt, int64_t sb, int64_t ss, const int64_t* position, int64_t window, int B,
+                int S, int32_t* ends, int32_t* starts, BoundsParams& p) {
   if (B < 0 || S <= 0) return fail(FSK_ERR_INVALID, "batch and positions must be positive");
   if (B > kMaxBatch) return fail(FSK_ERR_UNSUPPORTED, "batch above 16384");
   if (!ends || ((mask || window >= 0) && !starts)) return fail(FSK_ERR_INVALID, "null output pointer");
-  if (B == 0) return FSK_OK;
-  BoundsParams p;
   memset(&p, 0, sizeof(p));
   p.position = position; p.window = window;
   p.B = B; p.S = S; p.ends = ends; p.starts = starts;
+  p.mask_kind = -1;
+  p.blocks = mask ? B : (int)cdiv(B, kBoundsThreads);
   if (mask) {
     if (position || window >= 0) return fail(FSK_ERR_INVALID, "a mask, or a position and window");
     const int size = mask_dt == FSK_BOOL ? 1 : mask_dt == FSK_E4M3 ? 0 : elem_bytes(mask_dt);
@@ -3375,18 +3569,73 @@ int run_bounds(const void* mask, int mask_dt, int64_t sb, int64_t ss, const int6
     if (!aligned(mask, size)) return fail(FSK_ERR_INVALID, "mask not aligned to its type");
     p.mask = (const uint8_t*)mask;
     p.m_sb = sb * size; p.m_ss = ss * size;
+    p.mask_kind = mask_dt;
   }
+  return FSK_OK;
+}
+
+int run_bounds(const void* mask, int mask_dt, int64_t sb, int64_t ss, const int64_t* position, int64_t window, int B,
+               int S, int32_t* ends, int32_t* starts, hipStream_t stream) {
+  BoundsParams p;
+  const int st = make_bounds(mask, mask_dt, sb, ss, position, window, B, S, ends, starts, p);
+  if (st != FSK_OK || B == 0) return st;
   (void)hipGetLastError();
-  const Launch l{stream, nullptr, nullptr};
-  const dim3 grid((unsigned)B), block(kBoundsThreads);
-  if (!mask) launch(position_bounds_kernel, dim3((unsigned)cdiv(B, kBoundsThreads)), block, 0, l, p);
-  else if (mask_dt == FSK_BOOL) launch(mask_bounds_kernel<kBool>, grid, block, 0, l, p);
-  else if (mask_dt == FSK_F16) launch(mask_bounds_kernel<kF16>, grid, block, 0, l, p);
-  else if (mask_dt == FSK_BF16) launch(mask_bounds_kernel<kBF16>, grid, block, 0, l, p);
-  else launch(mask_bounds_kernel<kF32>, grid, block, 0, l, p);
+  launch(bounds_kernel, dim3((unsigned)p.blocks), dim3(kBoundsThreads), 0, Launch{stream, nullptr, nullptr}, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(FSK_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(e));
   return FSK_OK;
+}
+
+// The HF attention function's fp8 decode: ranges and maxima, then the
+// quantising decode kernels.
+struct QuantDecode {
+  const void *q, *k, *v;
+  int64_t numel[3];
+  const void* mask; int mask_dt; int64_t m_sb, m_ss;
+  const int64_t* position; int64_t window;
+};
+int64_t quant_ws_bytes(int B) { return align256(3 * kAmaxMax * 4) + align256(8 * (int64_t)B); }
+
+int run_quant_decode(const QuantDecode& a, Common c) {
+  if (c.q_dt != c.kv_dt || (c.q_dt != FSK_F16 && c.q_dt != FSK_BF16))
+    return fail(FSK_ERR_UNSUPPORTED, "q, k and v must be f16 or bf16, of one type");
+  if (c.Hkv > 0 && c.Hq > 16 * c.Hkv) return fail(FSK_ERR_UNSUPPORTED, "more than 16 query heads per KV head");
+  const int64_t own = quant_ws_bytes(std::max(c.B, 0));
+  if (!c.ws || c.ws_bytes < own || !aligned(c.ws, 256))
+    return fail(FSK_ERR_WORKSPACE, "workspace missing, unaligned or smaller than fsk_decode_dense_fp8_workspace_bytes()");
+  uint8_t* ws = (uint8_t*)c.ws;
+  uint32_t* part = (uint32_t*)ws;
+  int32_t* ends = (int32_t*)(ws + align256(3 * kAmaxMax * 4));
+  int32_t* starts = a.mask || a.window >= 0 ? ends + c.B : nullptr;
+  c.ws = ws + own;
+  c.ws_bytes -= own;
+  c.lens = ends;
+  c.starts = starts;
+  QuantPre pre;
+  BoundsParams& bp = pre.bp;
+  const int st = make_bounds(a.mask, a.mask_dt, a.m_sb, a.m_ss, a.position, a.window, c.B, (int)c.kv_extent, ends, starts, bp);
+  if (st != FSK_OK) return st;
+  QuantParams& qp = pre.qp;
+  memset(&qp, 0, sizeof(qp));
+  qp.part = part;
+  const void* src[3] = {a.q, a.k, a.v};
+  uint32_t grid = 0;
+  for (int i = 0; i < 3; ++i) {
+    if (!src[i]) return fail(FSK_ERR_INVALID, "null tensor pointer");
+    if (a.numel[i] <= 0) return fail(FSK_ERR_INVALID, "empty tensor");
+    if (a.numel[i] >= kMaxStride) return fail(FSK_ERR_UNSUPPORTED, "tensor above 2^40 elements");
+    if (!aligned(src[i], 16)) return fail(FSK_ERR_INVALID, "tensors must be 16-byte aligned");
+    QuantTensor& t = qp.t[i];
+    t.src = (const uint8_t*)src[i];
+    t.n = a.numel[i];
+    t.blk0 = grid;
+    t.nblk = (uint32_t)std::min<int64_t>(std::max<int64_t>(cdiv(t.n, (int64_t)kQuantThreads * kQuantStep), 1), kAmaxMax);
+    grid += t.nblk;
+  }
+  pre.grid = (unsigned)bp.blocks + grid;
+  pre.dt = c.q_dt;
+  c.pre = &pre;
+  return run_decode(c);  // (launches it once every check has passed)
 }
 
 }  // namespace
@@ -3759,6 +4008,39 @@ int fsk_decode_dense(const void* q, int64_t q_stride_b, int64_t q_stride_h, cons
   c.q_dt = q_dtype; c.kv_dt = kv_dtype; c.o_dt = out_dtype; c.sm_scale = sm_scale;
   c.ws = workspace; c.ws_bytes = workspace_bytes; c.chunk = chunk_tokens; c.stream = (hipStream_t)stream;
   return run_decode(c);
+}
+
+int64_t fsk_decode_dense_fp8_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                             int64_t max_seqlen, int chunk_tokens) {
+  const int64_t n = fsk_workspace_bytes(FSK_LAYOUT_DENSE, batch, num_q_heads, num_kv_heads, head_dim, max_seqlen, 16,
+                                        chunk_tokens);
+  return n < 0 ? n : n + quant_ws_bytes(batch);
+}
+
+int fsk_decode_dense_fp8(const void* q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_numel, const void* k,
+                         int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_t, int64_t k_numel, const void* v,
+                         int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_t, int64_t v_numel,
+                         int64_t max_seqlen, const void* mask, int mask_dtype, int64_t mask_stride_b,
+                         int64_t mask_stride_s, const int64_t* position, int64_t window, void* out,
+                         int64_t o_stride_b, int64_t o_stride_h, int batch, int num_q_heads, int num_kv_heads,
+                         int head_dim, int dtype, int out_dtype, float sm_scale, void* workspace,
+                         int64_t workspace_bytes, int chunk_tokens, void* stream) {
+  if (max_seqlen <= 0 || max_seqlen >= ((int64_t)1 << 31)) return fail(FSK_ERR_INVALID, "max_seqlen must be positive");
+  Common c;
+  memset(&c, 0, sizeof(c));
+  c.layout = FSK_LAYOUT_DENSE;
+  c.q = q; c.q_sb = q_stride_b; c.q_sh = q_stride_h;
+  c.k = k; c.k_s0 = k_stride_b; c.k_sh = k_stride_h; c.k_st = k_stride_t;
+  c.v = v; c.v_s0 = v_stride_b; c.v_sh = v_stride_h; c.v_st = v_stride_t;
+  c.kv_extent = max_seqlen;
+  c.sink_mode = FSK_SINK_LINEAR;
+  c.out = out; c.o_sb = o_stride_b; c.o_sh = o_stride_h;
+  c.B = batch; c.Hq = num_q_heads; c.Hkv = num_kv_heads; c.D = head_dim;
+  c.q_dt = c.kv_dt = dtype; c.o_dt = out_dtype; c.sm_scale = sm_scale;
+  c.ws = workspace; c.ws_bytes = workspace_bytes; c.chunk = chunk_tokens; c.stream = (hipStream_t)stream;
+  const QuantDecode a{q, k, v, {q_numel, k_numel, v_numel}, mask, mask_dtype, mask_stride_b, mask_stride_s, position,
+                      window};
+  return run_quant_decode(a, c);
 }
 
 int fsk_paged_gather(const void* pool, int64_t stride_p, int64_t stride_h, int64_t stride_t,

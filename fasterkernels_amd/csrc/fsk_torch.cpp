@@ -427,10 +427,42 @@ void kv_write(const at::Tensor& k_in, const at::Tensor& v_in, const at::Tensor& 
 // ---------------------------------------------------------------------------
 // Attended range of an HF decode step (fskernels.hip.hf)
 // ---------------------------------------------------------------------------
-// (ends, starts) int32 [B] for a batch of B sequences over S positions, from
-// the last query's row of a [B or 1, heads, queries, >= S] mask, else from the
-// last entry of cache_position (int64), else S, with an optional window
-// (starts is undefined without a mask and window).
+// The range's source: the last query's row of a [B or 1, heads, queries, >= S]
+// mask, else the last entry of cache_position (int64), else all S positions;
+// without a mask, an optional window.
+struct Range {
+  const void* mask = nullptr;
+  int mask_dt = FSK_F32;
+  int64_t m_sb = 0, m_ss = 0;
+  const int64_t* position = nullptr;
+  int64_t window = -1;
+};
+Range decode_range(int64_t B, int64_t S, const c10::optional<at::Tensor>& mask,
+                   const c10::optional<at::Tensor>& position, c10::optional<int64_t> window, const c10::Device& dev) {
+  Range r;
+  if (mask && mask->defined()) {
+    on_device(*mask, "attention_mask", dev);
+    if (mask->dim() != 4 || mask->size(1) < 1 || mask->size(2) < 1 || (mask->size(0) != B && mask->size(0) != 1) ||
+        (mask->size(3) < S && mask->size(3) != 1))
+      raise(kRuntime, "attention_mask must be [" + std::to_string(B) + ", heads, queries, >= " + std::to_string(S) +
+                          "], got " + shape_str(*mask));
+    r.mask_dt = mask->scalar_type() == at::kBool ? FSK_BOOL : dtype_code(mask->scalar_type(), "attention_mask");
+    r.m_sb = mask->size(0) == 1 ? 0 : mask->stride(0);
+    r.m_ss = mask->size(3) == 1 ? 0 : mask->stride(3);
+    r.mask = static_cast<const char*>(mask->data_ptr()) + (mask->size(2) - 1) * mask->stride(2) * mask->element_size();
+    return r;
+  }
+  if (position && position->defined()) {
+    on_device(*position, "cache_position", dev);
+    if (position->scalar_type() != at::kLong || position->dim() != 1 || position->numel() < 1)
+      raise(FSK_ERR_INVALID, "cache_position must be a non-empty int64 vector");
+    r.position = position->data_ptr<int64_t>() + (position->numel() - 1) * position->stride(0);
+  }
+  if (window) r.window = std::max<int64_t>(*window, 0);
+  return r;
+}
+
+// (ends, starts) int32 [B]; starts is undefined without a mask and window.
 std::pair<at::Tensor, c10::optional<at::Tensor>> bounds(const at::Tensor& like, int64_t B, int64_t S,
                                                         const c10::optional<at::Tensor>& mask,
                                                         const c10::optional<at::Tensor>& position,
@@ -438,32 +470,49 @@ std::pair<at::Tensor, c10::optional<at::Tensor>> bounds(const at::Tensor& like, 
   on_gpu(like, "query_states");
   const c10::Device dev = like.device();
   const c10::DeviceGuard guard(dev);
+  const Range r = decode_range(B, S, mask, position, window, dev);
   const at::Tensor out = at::empty({2, B}, like.options().dtype(at::kInt));
   int32_t* ends = out.data_ptr<int32_t>();
-  const void* mp = nullptr;
-  int md = FSK_F32;
-  int64_t sb = 0, ss = 0;
-  const int64_t* pp = nullptr;
-  if (mask && mask->defined()) {
-    on_device(*mask, "attention_mask", dev);
-    if (mask->dim() != 4 || mask->size(1) < 1 || mask->size(2) < 1 || (mask->size(0) != B && mask->size(0) != 1) ||
-        (mask->size(3) < S && mask->size(3) != 1))
-      raise(kRuntime, "attention_mask must be [" + std::to_string(B) + ", heads, queries, >= " + std::to_string(S) +
-                          "], got " + shape_str(*mask));
-    md = mask->scalar_type() == at::kBool ? FSK_BOOL : dtype_code(mask->scalar_type(), "attention_mask");
-    sb = mask->size(0) == 1 ? 0 : mask->stride(0);
-    ss = mask->size(3) == 1 ? 0 : mask->stride(3);
-    mp = static_cast<const char*>(mask->data_ptr()) + (mask->size(2) - 1) * mask->stride(2) * mask->element_size();
-  } else if (position && position->defined()) {
-    on_device(*position, "cache_position", dev);
-    if (position->scalar_type() != at::kLong || position->dim() != 1 || position->numel() < 1)
-      raise(FSK_ERR_INVALID, "cache_position must be a non-empty int64 vector");
-    pp = position->data_ptr<int64_t>() + (position->numel() - 1) * position->stride(0);
-  }
-  const bool with_starts = mp || window;
-  check(fsk_decode_bounds(mp, md, sb, ss, pp, !mp && window ? std::max<int64_t>(*window, 0) : -1, (int)B, (int)S, ends,
+  const bool with_starts = r.mask || r.window >= 0;
+  check(fsk_decode_bounds(r.mask, r.mask_dt, r.m_sb, r.m_ss, r.position, r.window, (int)B, (int)S, ends,
                           with_starts ? ends + B : nullptr, stream_ptr(stream)));
   return {out.select(0, 0), with_starts ? c10::optional<at::Tensor>(out.select(0, 1)) : c10::nullopt};
+}
+
+// The fp8 attention hook's decode (triton_gqa_decode_hf_fp8.py:230-283): q
+// [B, Hq, 1, D] and k/v [>= B, Hkv, S, D] of one 16-bit type, quantised per
+// tensor on the way.  Tensors with gaps or unaligned rows are packed first.
+at::Tensor dense_fp8(const at::Tensor& q_in, const at::Tensor& k_in, const at::Tensor& v_in,
+                     const c10::optional<at::Tensor>& mask, const c10::optional<at::Tensor>& position,
+                     c10::optional<int64_t> window, c10::optional<double> sm_scale, int64_t chunk_tokens,
+                     int64_t stream) {
+  on_gpu(q_in, "q");
+  if (q_in.dim() != 4 || q_in.size(2) != 1) raise(FSK_ERR_INVALID, "q must be [batch, num_q_heads, 1, head_dim], got " + shape_str(q_in));
+  const c10::Device dev = q_in.device();
+  const c10::DeviceGuard guard(dev);
+  auto packed = [](const at::Tensor& t) {
+    const at::Tensor r = rows16(t);
+    return r.is_non_overlapping_and_dense() ? r : r.clone(at::MemoryFormat::Contiguous);
+  };
+  on_device(k_in, "k_cache", dev);
+  on_device(v_in, "v_cache", dev);
+  if (k_in.dim() != 4 || v_in.sizes() != k_in.sizes() || k_in.size(3) != q_in.size(3) || k_in.size(0) < q_in.size(0))
+    raise(FSK_ERR_INVALID, "k_cache / v_cache shapes disagree with q");
+  if (k_in.scalar_type() != q_in.scalar_type() || v_in.scalar_type() != q_in.scalar_type())
+    raise(FSK_ERR_UNSUPPORTED, "q, k and v must have one dtype");
+  const at::Tensor q = packed(q_in), k = packed(k_in), v = packed(v_in);
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(3), Hkv = k.size(1), S = k.size(2);
+  const Range r = decode_range(B, S, mask, position, window, dev);
+  const at::Tensor out = at::empty({B, Hq, D}, q.options());
+  const int64_t nbytes = fsk_decode_dense_fp8_workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)D, S, (int)chunk_tokens);
+  const at::Tensor ws = workspace(nbytes, q);
+  const int dt = dtype_code(q.scalar_type(), "q");
+  check(fsk_decode_dense_fp8(q.data_ptr(), q.stride(0), q.stride(1), q.numel(), k.data_ptr(), k.stride(0), k.stride(1),
+                             k.stride(2), k.numel(), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), v.numel(), S,
+                             r.mask, r.mask_dt, r.m_sb, r.m_ss, r.position, r.window, out.data_ptr(), out.stride(0),
+                             out.stride(1), (int)B, (int)Hq, (int)Hkv, (int)D, dt, dt, softmax_scale(sm_scale, D),
+                             ws.data_ptr(), nbytes, (int)chunk_tokens, stream_ptr(stream)));
+  return out;
 }
 
 // ---------------------------------------------------------------------------
@@ -534,6 +583,8 @@ PYBIND11_MODULE(_fsk_torch, m) {
         py::arg("sink_mode"), py::arg("sm_scale"), py::arg("chunk_tokens"), py::arg("stream"));
   m.def("bounds", &bounds, py::arg("like"), py::arg("batch"), py::arg("positions"), py::arg("mask"),
         py::arg("cache_position"), py::arg("window"), py::arg("stream"));
+  m.def("dense_fp8", &dense_fp8, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("mask"), py::arg("cache_position"),
+        py::arg("window"), py::arg("sm_scale"), py::arg("chunk_tokens"), py::arg("stream"));
   m.def("quantize", &quantize, py::arg("tensors"), py::arg("stream"));
   m.def("kv_write", &kv_write, py::arg("k"), py::arg("v"), py::arg("k_pool"), py::arg("v_pool"), py::arg("slot_mapping"),
         py::arg("k_scale"), py::arg("v_scale"), py::arg("block_table"), py::arg("bt_updates"), py::arg("stream"));

@@ -66,6 +66,9 @@ SIGNATURES = {
     "fsk_paged_gather": (_I, [_P, _L, _L, _L, _P, _L, _I, _P, _I, _I, _I, _I, _I, _I, _P, _P]),
     "fsk_paged_write": (_I, [_P, _L, _L, _P, _L, _L, _P, _L, _P, _L, _L, _L, _P, _L, _L, _L, _I, _I,
                              _I, _I, _I, _I, _P, _P, _P, _L, _P, _L, _P]),
+    "fsk_decode_dense_fp8_workspace_bytes": (_L, [_I, _I, _I, _I, _L, _I]),
+    "fsk_decode_dense_fp8": (_I, [_P, _L, _L, _L, _P, _L, _L, _L, _L, _P, _L, _L, _L, _L, _L, _P, _I, _L, _L, _P, _L,
+                                  _P, _L, _L, _I, _I, _I, _I, _I, _I, _F, _P, _L, _I, _P]),
     "fsk_decode_bounds": (_I, [_P, _I, _L, _L, _P, _L, _I, _I, _P, _P, _P]),
     "fsk_quantize_workspace_bytes": (_L, [_I]),
     "fsk_quantize_e4m3": (_I, [_I, _P, _P, _I, _P, _P, _P, _L, _P]),

@@ -215,6 +215,14 @@ def flash_decode_gqa_varlen(q, k_varlen, v_varlen, cu_seqlens_k, s_aux=None, *,
 # ---------------------------------------------------------------------------
 # dense (HF static cache)
 # ---------------------------------------------------------------------------
+def _split_hint(S, num_splits) -> int:
+    """chunk_tokens for at least num_splits parts per sequence of S tokens:
+    chunks of at most ceil(S / num_splits), rounded up to 32 (0: no hint)."""
+    if not num_splits or num_splits <= 1:
+        return 0
+    return -max(32, -(-math.ceil(S / num_splits) // 32) * 32)
+
+
 def _dense(q, k_cache, v_cache, cache_lens, start_k_offsets, num_splits, *, q_scale=None,
            k_scale=None, v_scale=None, out_dtype=None, s_aux=None, sink_mode="linear",
            sm_scale=None, chunk_tokens=0):
@@ -222,9 +230,7 @@ def _dense(q, k_cache, v_cache, cache_lens, start_k_offsets, num_splits, *, q_sc
         _on_gpu(k_cache, "k_cache")
         if k_cache.dim() != 4:
             raise ValueError("k_cache must be [batch, num_kv_heads, max_seqlen, head_dim]")
-        S = k_cache.shape[2]
-        # at least num_splits parts per sequence: chunks of at most this size
-        chunk_tokens = -max(32, -(-math.ceil(S / num_splits) // 32) * 32)
+        chunk_tokens = _split_hint(k_cache.shape[2], num_splits)
     return nat.ext().dense(q, k_cache, v_cache, cache_lens, start_k_offsets, s_aux, _scale_tensor(q_scale, q),
                            _scale_tensor(k_scale, q), _scale_tensor(v_scale, q), _out_code(out_dtype),
                            _sink_mode(sink_mode), _sm(sm_scale), int(chunk_tokens), _stream(q))
@@ -243,6 +249,15 @@ def flash_decode_gqa_hf_dense_optimized(q, k_cache, v_cache, cache_lens, start_k
     n = _DECODE_NUM_SPLITS if num_splits is None else num_splits
     return _dense(q, k_cache, v_cache, cache_lens, start_k_offsets, n, s_aux=s_aux,
                   sink_mode=sink_mode, sm_scale=sm_scale)
+
+
+def decode_quantizing_to_fp8(q, k, v, mask, cache_position, window, sm_scale):
+    """``flash_decode_gqa_hf_fp8`` of the quantised ``q`` [B, Hq, 1, D], ``k``
+    and ``v`` [B, Hkv, S, D] (16-bit, one dtype, at most 16 query heads per KV
+    head), quantised on the way to the matrix cores: no codes are stored.  The
+    attended ranges come from the mask or position (fskernels.hip.hf)."""
+    return nat.ext().dense_fp8(q, k, v, mask, cache_position, window, _sm(sm_scale),
+                               _split_hint(k.shape[2], _DECODE_NUM_SPLITS_FP8), _stream(q))
 
 
 def flash_decode_gqa_hf_fp8(q_fp8, k_cache_fp8, v_cache_fp8, cache_lens, scale_q, scale_k,

@@ -46,8 +46,8 @@ import torch
 
 from fasterkernels_amd import native as nat
 
-from .decode import (_on_gpu, _stream, flash_decode_gqa_hf_dense_optimized, flash_decode_gqa_hf_fp8,
-                     quantize_each_to_fp8)
+from .decode import (_on_gpu, _stream, decode_quantizing_to_fp8, flash_decode_gqa_hf_dense_optimized,
+                     flash_decode_gqa_hf_fp8, quantize_each_to_fp8)
 
 _MASK_DTYPES = (torch.bool, torch.float16, torch.bfloat16, torch.float32)
 
@@ -89,13 +89,19 @@ def _decode_bounds(query_states: torch.Tensor, key_states: torch.Tensor, attenti
     cache_position = kwargs.get("cache_position")
     if cache_position is not None:
         attention_mask = None
-        kernel = cache_position.dtype is torch.int64 and cache_position.dim() == 1 and cache_position.is_cuda
-    else:
-        kernel = attention_mask is None or (attention_mask.dtype in _MASK_DTYPES and attention_mask.dim() == 4)
-    if not kernel or not 0 < S < 1 << 31:
+    if not _kernel_bounds(S, attention_mask, cache_position):
         return _torch_bounds(bsz, S, query_states.device, attention_mask, cache_position, window)
     return nat.ext().bounds(query_states, bsz, S, attention_mask, cache_position,
                             None if window is None else int(window), _stream(query_states))
+
+
+def _kernel_bounds(S, attention_mask, cache_position) -> bool:
+    """Whether the kernels read the range from this mask or position."""
+    if not 0 < S < 1 << 31:
+        return False
+    if cache_position is not None:
+        return cache_position.dtype is torch.int64 and cache_position.dim() == 1 and cache_position.is_cuda
+    return attention_mask is None or (attention_mask.dtype in _MASK_DTYPES and attention_mask.dim() == 4)
 
 
 def _torch_bounds(bsz, S, dev, attention_mask, cache_position, window):
@@ -141,8 +147,20 @@ def custom_hf_decode_attention_forward_fp8(module: torch.nn.Module, query_states
                                            attention_mask, scaling: float, dropout: float = 0.0, **kwargs):
     """FP8 variant: Q, K and V are quantised per call with per-tensor scales
     (the codes of quantize_to_fp8 of their fp32 values, as
-    triton_gqa_decode_hf_fp8.py:268-273 takes them) and decoded by the e4m3
-    kernels; the output keeps the query dtype."""
+    triton_gqa_decode_hf_fp8.py:268-273 takes them); the output keeps the
+    query dtype.  16-bit tensors are quantised inside the decode kernels, any
+    others (and more than 16 query heads per KV head, where K and V are read
+    several times) by a pass of their own."""
+    q, k, v = query_states, key_states, value_states
+    if (q.shape[2] == 1 and q.dtype in (torch.float16, torch.bfloat16) and k.dtype is q.dtype and v.dtype is q.dtype
+            and q.is_cuda and k.is_cuda and v.is_cuda and 0 < q.numel() and 0 < k.numel()
+            and q.shape[1] <= 16 * k.shape[1]):
+        position = kwargs.get("cache_position")
+        mask = attention_mask if position is None else None
+        if _kernel_bounds(k.shape[2], mask, position):
+            window = kwargs.get("sliding_window")
+            return decode_quantizing_to_fp8(q, k, v, mask, position, None if window is None else int(window),
+                                            scaling), None
     bounds = _decode_bounds(query_states, key_states, attention_mask, kwargs)
     if bounds is None:
         return native_eager_attention_forward(module, query_states, key_states, value_states,

@@ -372,6 +372,29 @@ FSK_API int fsk_quantize_e4m3(int count, const void *const *src, const int64_t *
                       void *const *dst, float *const *scale,
                       void *workspace, int64_t workspace_bytes, void *stream);
 
+/* Dense decode of f16 / bf16 Q, K and V that quantises them per tensor on the
+ * way: the result of fsk_decode_bounds, fsk_quantize_e4m3 of Q, K and V and
+ * fsk_decode_dense of the codes, without storing the codes.
+ * Replaces: fskernels/triton/triton_gqa_decode_hf_fp8.py:230-283.
+ * q [B, Hq, D], k/v [>= B, Hkv, S, D] of one dtype, each a dense tensor of
+ * *_numel elements starting at its pointer (the scales cover all of them), at
+ * most 16 query heads per KV head.  The attended ranges come from the mask,
+ * position and window as fsk_decode_bounds takes them.  The workspace holds
+ * fsk_decode_dense_fp8_workspace_bytes(...) bytes. */
+FSK_API int64_t fsk_decode_dense_fp8_workspace_bytes(int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                                     int64_t max_seqlen, int chunk_tokens);
+FSK_API int fsk_decode_dense_fp8(const void *q, int64_t q_stride_b, int64_t q_stride_h, int64_t q_numel,
+                                 const void *k, int64_t k_stride_b, int64_t k_stride_h, int64_t k_stride_t,
+                                 int64_t k_numel,
+                                 const void *v, int64_t v_stride_b, int64_t v_stride_h, int64_t v_stride_t,
+                                 int64_t v_numel, int64_t max_seqlen,
+                                 const void *mask, int mask_dtype, int64_t mask_stride_b, int64_t mask_stride_s,
+                                 const int64_t *position, int64_t window,
+                                 void *out, int64_t o_stride_b, int64_t o_stride_h,
+                                 int batch, int num_q_heads, int num_kv_heads, int head_dim,
+                                 int dtype, int out_dtype, float sm_scale,
+                                 void *workspace, int64_t workspace_bytes, int chunk_tokens, void *stream);
+
 /* Tuning knobs for benchmarking sweeps:
  *   "chunk_tokens"        fixed split size in tokens (0: chosen on the device)
  *   "waves_per_cu"        largest persistent grid, workgroups per CU (default

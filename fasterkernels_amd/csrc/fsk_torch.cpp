@@ -15,6 +15,7 @@
 // tensors' device); the device guard makes that device current for the call.
 #include <torch/extension.h>
 
+#include <c10/core/Allocator.h>
 #include <c10/core/DeviceGuard.h>
 
 #include <algorithm>
@@ -163,9 +164,15 @@ bool score_tensor(const c10::optional<at::Tensor>& s, int64_t B, int64_t Hq, at:
   return true;
 }
 
-at::Tensor workspace(int64_t nbytes, const at::Tensor& like) {
+// Scratch memory of one call on the current device and stream, from the
+// allocator that at::empty has just given `out` its memory from (torch's
+// caching allocator: stream-ordered reuse, graph pools), without making a
+// tensor of it (0.23 us a call instead of 0.70).
+c10::DataPtr workspace(int64_t nbytes, const at::Tensor& out) {
   if (nbytes < 0) check((int)nbytes);
-  return at::empty({nbytes}, like.options().dtype(at::kByte));
+  c10::Allocator* allocator = out.storage().allocator();
+  if (!allocator) raise(kRuntime, "the output tensor has no allocator");
+  return allocator->allocate((size_t)nbytes);
 }
 
 void* stream_ptr(int64_t stream) { return reinterpret_cast<void*>(static_cast<intptr_t>(stream)); }
@@ -211,7 +218,7 @@ at::Tensor paged(const at::Tensor& q_in, const at::Tensor& k_pool, const at::Ten
     if (extra < 0) check((int)extra);
     nbytes += extra;
   }
-  const at::Tensor ws = workspace(nbytes, q);
+  const c10::DataPtr ws = workspace(nbytes, out);
   const int qd = dtype_code(q.scalar_type(), "q"), kd = dtype_code(k.scalar_type(), "k_pool");
   const int od = dtype_code(out.scalar_type(), "out_dtype");
   const float scl = softmax_scale(sm_scale, D);
@@ -225,14 +232,14 @@ at::Tensor paged(const at::Tensor& q_in, const at::Tensor& k_pool, const at::Ten
                           k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), bt.data_ptr<int32_t>(),
                           bt.stride(0), (int)max_blocks, lens.data_ptr<int32_t>(), (int)P, (int)PS, sp,
                           (int)sink_mode, ksp, vsp, out.data_ptr(), out.stride(0), out.stride(1), (int)B, (int)Hq,
-                          (int)Hkv, (int)D, qd, kd, od, scl, ws.data_ptr(), nbytes, (int)chunk_tokens,
+                          (int)Hkv, (int)D, qd, kd, od, scl, ws.get(), nbytes, (int)chunk_tokens,
                           stream_ptr(stream));
   } else {
     st = fsk_decode_paged_scores(q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1),
                                  k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2),
                                  bt.data_ptr<int32_t>(), bt.stride(0), (int)max_blocks, lens.data_ptr<int32_t>(),
                                  (int)P, (int)PS, sp, (int)sink_mode, ksp, vsp, out.data_ptr(), out.stride(0),
-                                 out.stride(1), (int)B, (int)Hq, (int)Hkv, (int)D, qd, kd, od, scl, ws.data_ptr(),
+                                 out.stride(1), (int)B, (int)Hq, (int)Hkv, (int)D, qd, kd, od, scl, ws.get(),
                                  nbytes, (int)chunk_tokens, scores->data_ptr(), (int)scores->size(2),
                                  stream_ptr(stream));
   }
@@ -272,7 +279,7 @@ at::Tensor varlen(const at::Tensor& q_in, const at::Tensor& k_varlen, const at::
     if (extra < 0) check((int)extra);
     nbytes += extra;
   }
-  const at::Tensor ws = workspace(nbytes, q);
+  const c10::DataPtr ws = workspace(nbytes, out);
   const int qd = dtype_code(q.scalar_type(), "q"), kd = dtype_code(k.scalar_type(), "k_varlen");
   const int od = dtype_code(out.scalar_type(), "out_dtype");
   const float scl = softmax_scale(sm_scale, D);
@@ -285,12 +292,12 @@ at::Tensor varlen(const at::Tensor& q_in, const at::Tensor& k_varlen, const at::
     st = entry(q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1),
                            v.data_ptr(), v.stride(0), v.stride(1), cu.data_ptr<int32_t>(), T, sp, (int)sink_mode, ksp,
                            vsp, out.data_ptr(), out.stride(0), out.stride(1), (int)B, (int)Hq, (int)Hkv, (int)D, qd,
-                           kd, od, scl, ws.data_ptr(), nbytes, (int)chunk_tokens, stream_ptr(stream));
+                           kd, od, scl, ws.get(), nbytes, (int)chunk_tokens, stream_ptr(stream));
   } else {
     st = fsk_decode_varlen_scores(q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1),
                                   v.data_ptr(), v.stride(0), v.stride(1), cu.data_ptr<int32_t>(), T, sp,
                                   (int)sink_mode, ksp, vsp, out.data_ptr(), out.stride(0), out.stride(1), (int)B,
-                                  (int)Hq, (int)Hkv, (int)D, qd, kd, od, scl, ws.data_ptr(), nbytes,
+                                  (int)Hq, (int)Hkv, (int)D, qd, kd, od, scl, ws.get(), nbytes,
                                   (int)chunk_tokens, scores->data_ptr(), (int)scores->size(2), stream_ptr(stream));
   }
   check(st);
@@ -328,7 +335,7 @@ at::Tensor dense(const at::Tensor& q_in, const at::Tensor& k_cache, const at::Te
   const at::Tensor out = at::empty({B, Hq, D}, q.options().dtype(out_dtype(out_code, q)));
   const int64_t nbytes =
       fsk_workspace_bytes(FSK_LAYOUT_DENSE, (int)B, (int)Hq, (int)Hkv, (int)D, S, 16, (int)chunk_tokens);
-  const at::Tensor ws = workspace(nbytes, q);
+  const c10::DataPtr ws = workspace(nbytes, out);
   const int st = fsk_decode_dense(
       q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), v.data_ptr(),
       v.stride(0), v.stride(1), v.stride(2), S, lens.data_ptr<int32_t>(),
@@ -336,7 +343,7 @@ at::Tensor dense(const at::Tensor& q_in, const at::Tensor& k_cache, const at::Te
       static_cast<const float*>(ptr_or_null(qs)), static_cast<const float*>(ptr_or_null(ks)),
       static_cast<const float*>(ptr_or_null(vs)), out.data_ptr(), out.stride(0), out.stride(1), (int)B, (int)Hq,
       (int)Hkv, (int)D, dtype_code(q.scalar_type(), "q"), dtype_code(k.scalar_type(), "k_cache"),
-      dtype_code(out.scalar_type(), "out_dtype"), softmax_scale(sm_scale, D), ws.data_ptr(), nbytes,
+      dtype_code(out.scalar_type(), "out_dtype"), softmax_scale(sm_scale, D), ws.get(), nbytes,
       (int)chunk_tokens, stream_ptr(stream));
   check(st);
   return out;
@@ -479,6 +486,42 @@ std::pair<at::Tensor, c10::optional<at::Tensor>> bounds(const at::Tensor& like, 
   return {out.select(0, 0), with_starts ? c10::optional<at::Tensor>(out.select(0, 1)) : c10::nullopt};
 }
 
+// The attention hook's decode (triton_gqa_decode_hf.py:218-258): q [B, Hq, 1,
+// D] over the dense cache k/v [>= B, Hkv, S, D], the range and the decode in
+// one call (the range stays in scratch memory).
+at::Tensor dense_hf(const at::Tensor& q_in, const at::Tensor& k_cache, const at::Tensor& v_cache,
+                    const c10::optional<at::Tensor>& mask, const c10::optional<at::Tensor>& position,
+                    c10::optional<int64_t> window, c10::optional<double> sm_scale, int64_t chunk_tokens,
+                    int64_t stream) {
+  on_gpu(q_in, "q");
+  if (q_in.dim() != 4 || q_in.size(2) != 1) raise(FSK_ERR_INVALID, "q must be [batch, num_q_heads, 1, head_dim], got " + shape_str(q_in));
+  const at::Tensor q = check_q(q_in.select(2, 0));
+  const c10::Device dev = q.device();
+  const c10::DeviceGuard guard(dev);
+  const at::Tensor k = kv_tensor(k_cache, "k_cache", dev, 4, "[batch, num_kv_heads, max_seqlen, head_dim]");
+  const at::Tensor v = kv_tensor(v_cache, "v_cache", dev, 4, "[batch, num_kv_heads, max_seqlen, head_dim]");
+  const int64_t B = q.size(0), Hq = q.size(1), D = q.size(2), Hkv = k.size(1), S = k.size(2);
+  if (v.sizes() != k.sizes() || k.size(3) != D || k.size(0) < B)
+    raise(FSK_ERR_INVALID, "k_cache / v_cache shapes disagree with q");
+  const Range r = decode_range(B, S, mask, position, window, dev);
+  const at::Tensor out = at::empty({B, Hq, D}, q.options());
+  int64_t nbytes = fsk_workspace_bytes(FSK_LAYOUT_DENSE, (int)B, (int)Hq, (int)Hkv, (int)D, S, 16, (int)chunk_tokens);
+  if (nbytes < 0) check((int)nbytes);
+  const c10::DataPtr ws = workspace(nbytes, out);  // (256-byte aligned, like every allocation)
+  const c10::DataPtr range = workspace(std::max<int64_t>(8 * B, 8), out);
+  int32_t* ends = static_cast<int32_t*>(range.get());
+  int32_t* starts = r.mask || r.window >= 0 ? ends + B : nullptr;
+  check(fsk_decode_bounds(r.mask, r.mask_dt, r.m_sb, r.m_ss, r.position, r.window, (int)B, (int)S, ends, starts,
+                          stream_ptr(stream)));
+  check(fsk_decode_dense(q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
+                         v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), S, ends, starts, nullptr,
+                         FSK_SINK_LINEAR, nullptr, nullptr, nullptr, out.data_ptr(), out.stride(0), out.stride(1),
+                         (int)B, (int)Hq, (int)Hkv, (int)D, dtype_code(q.scalar_type(), "q"),
+                         dtype_code(k.scalar_type(), "k_cache"), dtype_code(out.scalar_type(), "out_dtype"),
+                         softmax_scale(sm_scale, D), ws.get(), nbytes, (int)chunk_tokens, stream_ptr(stream)));
+  return out;
+}
+
 // The fp8 attention hook's decode (triton_gqa_decode_hf_fp8.py:230-283): q
 // [B, Hq, 1, D] and k/v [>= B, Hkv, S, D] of one 16-bit type, quantised per
 // tensor on the way.  Tensors with gaps or unaligned rows are packed first.
@@ -505,13 +548,13 @@ at::Tensor dense_fp8(const at::Tensor& q_in, const at::Tensor& k_in, const at::T
   const Range r = decode_range(B, S, mask, position, window, dev);
   const at::Tensor out = at::empty({B, Hq, D}, q.options());
   const int64_t nbytes = fsk_decode_dense_fp8_workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)D, S, (int)chunk_tokens);
-  const at::Tensor ws = workspace(nbytes, q);
+  const c10::DataPtr ws = workspace(nbytes, out);
   const int dt = dtype_code(q.scalar_type(), "q");
   check(fsk_decode_dense_fp8(q.data_ptr(), q.stride(0), q.stride(1), q.numel(), k.data_ptr(), k.stride(0), k.stride(1),
                              k.stride(2), k.numel(), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), v.numel(), S,
                              r.mask, r.mask_dt, r.m_sb, r.m_ss, r.position, r.window, out.data_ptr(), out.stride(0),
                              out.stride(1), (int)B, (int)Hq, (int)Hkv, (int)D, dt, dt, softmax_scale(sm_scale, D),
-                             ws.data_ptr(), nbytes, (int)chunk_tokens, stream_ptr(stream)));
+                             ws.get(), nbytes, (int)chunk_tokens, stream_ptr(stream)));
   return out;
 }
 
@@ -548,8 +591,8 @@ std::vector<std::pair<at::Tensor, at::Tensor>> quantize(const std::vector<at::Te
     res.emplace_back(codes, sc);
   }
   const int64_t nbytes = fsk_quantize_workspace_bytes(n);
-  const at::Tensor ws = workspace(nbytes, xs[0]);
-  check(fsk_quantize_e4m3(n, sp, numel, dtype_code(xs[0].scalar_type(), "x"), dp, cp, ws.data_ptr(), nbytes,
+  const c10::DataPtr ws = workspace(nbytes, res[0].first);
+  check(fsk_quantize_e4m3(n, sp, numel, dtype_code(xs[0].scalar_type(), "x"), dp, cp, ws.get(), nbytes,
                           stream_ptr(stream)));
   return res;
 }
@@ -583,6 +626,8 @@ PYBIND11_MODULE(_fsk_torch, m) {
         py::arg("sink_mode"), py::arg("sm_scale"), py::arg("chunk_tokens"), py::arg("stream"));
   m.def("bounds", &bounds, py::arg("like"), py::arg("batch"), py::arg("positions"), py::arg("mask"),
         py::arg("cache_position"), py::arg("window"), py::arg("stream"));
+  m.def("dense_hf", &dense_hf, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("mask"), py::arg("cache_position"),
+        py::arg("window"), py::arg("sm_scale"), py::arg("chunk_tokens"), py::arg("stream"));
   m.def("dense_fp8", &dense_fp8, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("mask"), py::arg("cache_position"),
         py::arg("window"), py::arg("sm_scale"), py::arg("chunk_tokens"), py::arg("stream"));
   m.def("quantize", &quantize, py::arg("tensors"), py::arg("stream"));

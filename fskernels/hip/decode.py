@@ -251,6 +251,13 @@ def flash_decode_gqa_hf_dense_optimized(q, k_cache, v_cache, cache_lens, start_k
                   sink_mode=sink_mode, sm_scale=sm_scale)
 
 
+def decode_hf(q, k, v, mask, cache_position, window, sm_scale):
+    """``flash_decode_gqa_hf_dense_optimized`` of ``q`` [B, Hq, 1, D] over the
+    range that the mask or position gives (fskernels.hip.hf), in one call."""
+    return nat.ext().dense_hf(q, k, v, mask, cache_position, window, _sm(sm_scale),
+                              _split_hint(k.shape[2], _DECODE_NUM_SPLITS), _stream(q))
+
+
 def decode_quantizing_to_fp8(q, k, v, mask, cache_position, window, sm_scale):
     """``flash_decode_gqa_hf_fp8`` of the quantised ``q`` [B, Hq, 1, D], ``k``
     and ``v`` [B, Hkv, S, D] (16-bit, one dtype, at most 16 query heads per KV

@@ -46,7 +46,7 @@ import torch
 
 from fasterkernels_amd import native as nat
 
-from .decode import (_on_gpu, _stream, decode_quantizing_to_fp8, flash_decode_gqa_hf_dense_optimized,
+from .decode import (_on_gpu, _stream, decode_hf, decode_quantizing_to_fp8, flash_decode_gqa_hf_dense_optimized,
                      flash_decode_gqa_hf_fp8, quantize_each_to_fp8)
 
 _MASK_DTYPES = (torch.bool, torch.float16, torch.bfloat16, torch.float32)
@@ -85,23 +85,29 @@ def _decode_bounds(query_states: torch.Tensor, key_states: torch.Tensor, attenti
         return None
     _on_gpu(query_states, "query_states")
     S = key_states.shape[2]
-    window = kwargs.get("sliding_window")
+    source = _range_source(query_states, key_states, attention_mask, kwargs)
+    if source is not None:
+        return nat.ext().bounds(query_states, bsz, S, *source, _stream(query_states))
     cache_position = kwargs.get("cache_position")
-    if cache_position is not None:
+    return _torch_bounds(bsz, S, query_states.device, attention_mask if cache_position is None else None,
+                         cache_position, kwargs.get("sliding_window"))
+
+
+def _range_source(query_states, key_states, attention_mask, kwargs):
+    """(mask, position, window) that the kernels take the range from, or None
+    where they do not read this mask or position type."""
+    S = key_states.shape[2]
+    position = kwargs.get("cache_position")
+    if not query_states.is_cuda or not 0 < S < 1 << 31:
+        return None
+    if position is not None:
         attention_mask = None
-    if not _kernel_bounds(S, attention_mask, cache_position):
-        return _torch_bounds(bsz, S, query_states.device, attention_mask, cache_position, window)
-    return nat.ext().bounds(query_states, bsz, S, attention_mask, cache_position,
-                            None if window is None else int(window), _stream(query_states))
-
-
-def _kernel_bounds(S, attention_mask, cache_position) -> bool:
-    """Whether the kernels read the range from this mask or position."""
-    if not 0 < S < 1 << 31:
-        return False
-    if cache_position is not None:
-        return cache_position.dtype is torch.int64 and cache_position.dim() == 1 and cache_position.is_cuda
-    return attention_mask is None or (attention_mask.dtype in _MASK_DTYPES and attention_mask.dim() == 4)
+        if not (position.dtype is torch.int64 and position.dim() == 1 and position.is_cuda):
+            return None
+    elif attention_mask is not None and not (attention_mask.dtype in _MASK_DTYPES and attention_mask.dim() == 4):
+        return None
+    window = kwargs.get("sliding_window")
+    return attention_mask, position, None if window is None else int(window)
 
 
 def _torch_bounds(bsz, S, dev, attention_mask, cache_position, window):
@@ -132,6 +138,10 @@ def custom_hf_decode_attention_forward(module: torch.nn.Module, query_states: to
     kernels over the dense cache, everything else on transformers' eager path.
     Returns (attn_output [B, Hq, D], None) on decode steps (reshaped by the
     caller exactly as eager's [B, 1, Hq, D])."""
+    if query_states.shape[2] == 1:
+        source = _range_source(query_states, key_states, attention_mask, kwargs)
+        if source is not None:
+            return decode_hf(query_states, key_states, value_states, *source, scaling), None
     bounds = _decode_bounds(query_states, key_states, attention_mask, kwargs)
     if bounds is None:
         return native_eager_attention_forward(module, query_states, key_states, value_states,
@@ -155,12 +165,9 @@ def custom_hf_decode_attention_forward_fp8(module: torch.nn.Module, query_states
     if (q.shape[2] == 1 and q.dtype in (torch.float16, torch.bfloat16) and k.dtype is q.dtype and v.dtype is q.dtype
             and q.is_cuda and k.is_cuda and v.is_cuda and 0 < q.numel() and 0 < k.numel()
             and q.shape[1] <= 16 * k.shape[1]):
-        position = kwargs.get("cache_position")
-        mask = attention_mask if position is None else None
-        if _kernel_bounds(k.shape[2], mask, position):
-            window = kwargs.get("sliding_window")
-            return decode_quantizing_to_fp8(q, k, v, mask, position, None if window is None else int(window),
-                                            scaling), None
+        source = _range_source(q, k, attention_mask, kwargs)
+        if source is not None:
+            return decode_quantizing_to_fp8(q, k, v, *source, scaling), None
     bounds = _decode_bounds(query_states, key_states, attention_mask, kwargs)
     if bounds is None:
         return native_eager_attention_forward(module, query_states, key_states, value_states,

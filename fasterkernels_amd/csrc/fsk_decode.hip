@@ -1682,14 +1682,13 @@ struct ReduceParams {
 
 constexpr int kReduceThreads = 256;
 
+// Rows h0 .. h0 + kRows - 1 (query heads) of sequence b.
 template <int D, int kOut, int kRows>
-__global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) {
-  // One workgroup per kRows query heads of a sequence (kRows > 1 for large
-  // batches of short sequences, whose rows have few partials each).  Thread
-  // t of row r = t / (256 / kRows) owns the float4 column d4 = t % (D/4) of
-  // unit group grp; group grp merges units grp, grp + kGroups, ... with an
-  // online LSE update, loading kPer units per round trip, and the groups
-  // combine through LDS.
+__device__ __forceinline__ void reduce_rows(const ReduceParams& p, int h0, int b) {
+  // Thread t of row r = t / (256 / kRows) owns the float4 column d4 = t %
+  // (D/4) of unit group grp; group grp merges units grp, grp + kGroups, ...
+  // with an online LSE update, loading kPer units per round trip, and the
+  // groups combine through LDS.
   constexpr int kD4 = D / 4;
   constexpr int kRowThreads = kReduceThreads / kRows;
   constexpr int kGroups = kRowThreads / kD4;
@@ -1702,8 +1701,7 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) 
   const int row = tid / kRowThreads;
   const int d4 = (tid - row * kRowThreads) % kD4;
   const int grp = (tid - row * kRowThreads) / kD4;
-  const int h = blockIdx.x * kRows + row;
-  const int b = blockIdx.y;
+  const int h = h0 + row;
   const int kvh = h / p.G;
   const int hg = h - kvh * p.G;
   // The sink and the sequence length are loaded with the unit range, not
@@ -1815,6 +1813,67 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) 
   } else {
     *(uint32_t __attribute__((ext_vector_type(2)))*)((bf16*)o + 4 * d4) =
         u32x2{pack_bf16x2(val[0], val[1]), pack_bf16x2(val[2], val[3])};
+  }
+}
+
+// One workgroup per (query head, sequence).
+template <int D, int kOut>
+__global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) {
+  reduce_rows<D, kOut, 1>(p, blockIdx.x, blockIdx.y);
+}
+
+// For many rows (more than the 2048 workgroups that fit the chip at once),
+// where starting a workgroup per row is what takes the time (~1 ns each: 16384
+// rows 15 us, and leaving most of them at once was slower still).  Workgroups
+// kLongGroups + i merge kManyRows rows of a sequence of few partials each; the
+// sequences of many partials among them keep a workgroup per row, dealt to
+// the first kLongGroups workgroups, which look them up in the plan (eight such
+// rows read through one CU: 64 sequences of 16 tokens and one of 32000, 44 us
+// instead of 28).  Step times before and after, fp16, us: 64 query heads on 4 KV
+// heads x 128, 128 x 300 tokens 31.0 -> 27.5, 65 x 2048 61.4 -> 55.2; 64 on 8 x
+// 64, 65 x 300 20.2 -> 16.1, 65 lognormal 90.9 -> 83.5; 32 on 8 x 128, 128 x 2048
+// 179.2 -> 165.6, varlen 199 x U[76,422] 50.4 -> 46.9, one sequence of 32000
+// among 64 of 16 34.4 -> 32.0.  At 512 to 2048 rows the two differ by -3 to +5 %
+// either way (64 lognormal 142.6 and 142.9), so one workgroup per row stays.
+template <int D>
+constexpr int kManyRows = D <= 128 ? 8 : 4;
+constexpr int kFewUnits = 16;    // partials of a sequence that count as few
+constexpr int kLongGroups = 512;
+template <int D, int kOut>
+__global__ __launch_bounds__(kReduceThreads) void reduce_many_kernel(ReduceParams p, int B, FastDiv per_seq) {
+  if ((int)blockIdx.x >= kLongGroups) {
+    const uint32_t i = blockIdx.x - kLongGroups;
+    const uint32_t b = fdiv(i, per_seq);  // per_seq = Hq / kManyRows workgroups of a sequence
+    if (p.plan[b + 1] - p.plan[b] > kFewUnits) return;
+    reduce_rows<D, kOut, kManyRows<D>>(p, (int)(i - b * per_seq.d) * kManyRows<D>, (int)b);
+    return;
+  }
+  __shared__ uint64_t s_long[kReduceThreads / kWave];  // the long ones of kReduceThreads sequences
+  int row = blockIdx.x;  // of the long sequences' rows, in order; then every kLongGroups-th
+  int before = 0;        // long sequences passed
+  for (int b0 = 0; b0 < B; b0 += kReduceThreads) {
+    const int b = b0 + (int)threadIdx.x;
+    const uint64_t is_long = __ballot(b < B && p.plan[min(b, B - 1) + 1] - p.plan[min(b, B - 1)] > kFewUnits);
+    if ((threadIdx.x & (kWave - 1)) == 0) s_long[threadIdx.x / kWave] = is_long;
+    __syncthreads();
+    int here = 0;
+#pragma unroll
+    for (int w = 0; w < kReduceThreads / kWave; ++w) here += __builtin_popcountll(s_long[w]);
+    here = uniform(here);
+    for (int k = row / p.Hq; k < before + here; row += kLongGroups, k = row / p.Hq) {
+      int left = k - before, w = 0;  // the left-th set bit of s_long
+      uint64_t m = s_long[0];
+      while (left >= __builtin_popcountll(m)) {
+        left -= __builtin_popcountll(m);
+        m = s_long[++w];
+      }
+      while (left-- > 0) m &= m - 1;
+      const int seq = uniform(b0 + w * kWave + __builtin_ctzll(m));
+      reduce_rows<D, kOut, 1>(p, row - k * p.Hq, seq);
+      __syncthreads();
+    }
+    before += here;
+    __syncthreads();
   }
 }
 
@@ -3052,29 +3111,31 @@ int dispatch_layout(int layout, bool scores, const Params& p, int grid, int q_dt
   return dispatch_qkv<D, kDense, false>(p, grid, q_dt, kv_dt, s);
 }
 
-template <int D, int kRows>
-void launch_reduce_rows(const ReduceParams& rp, int B, int o_dt, const Launch& s) {
-  dim3 grid(rp.Hq / kRows, B);
-  dim3 block(kReduceThreads);
-  if (o_dt == FSK_F16) launch(reduce_kernel<D, kF16, kRows>, grid, block, 0, s, rp);
-  else if (o_dt == FSK_BF16) launch(reduce_kernel<D, kBF16, kRows>, grid, block, 0, s, rp);
-  else launch(reduce_kernel<D, kF32, kRows>, grid, block, 0, s, rp);
-}
-
-// Four query heads per workgroup when the batch has at least twice as many
-// sequences as the split has chunks (a few partials per row): a quarter of
-// the workgroups, each merging 8 units per round trip and row (D = 128).
-template <int D>
-void launch_reduce(const ReduceParams& rp, int B, int o_dt, bool rows4, const Launch& s) {
-  if (rows4 && rp.Hq % 4 == 0 && !rp.scores) launch_reduce_rows<D, 4>(rp, B, o_dt, s);
-  else launch_reduce_rows<D, 1>(rp, B, o_dt, s);
-}
-
 FastDiv make_fastdiv(uint32_t d) {
   uint32_t l = 0;
   while (((uint64_t)1 << l) < d) ++l;
   const uint64_t two_s = (uint64_t)1 << (31 + l);
   return FastDiv{d, (uint32_t)((two_s + d - 1) / d), 31 + l};
+}
+
+template <int D, int kOut>
+void launch_reduce_out(const ReduceParams& rp, int B, bool many, const Launch& s) {
+  if (many)
+    launch(reduce_many_kernel<D, kOut>, dim3((unsigned)(kLongGroups + (int64_t)rp.Hq / kManyRows<D> * B)),
+           dim3(kReduceThreads), 0, s, rp, B, make_fastdiv((uint32_t)(rp.Hq / kManyRows<D>)));
+  else
+    launch(reduce_kernel<D, kOut>, dim3(rp.Hq, B), dim3(kReduceThreads), 0, s, rp);
+}
+
+// More rows than workgroups fit at once (2048 of 256 threads on 256 CUs): see
+// reduce_many_kernel.
+template <int D>
+void launch_reduce(const ReduceParams& rp, int B, int o_dt, const Launch& s) {
+  const int64_t rows = (int64_t)rp.Hq * B;
+  const bool many = rows > 2048 && rows < ((int64_t)1 << 31) - 4096 && rp.Hq % kManyRows<D> == 0 && !rp.scores;
+  if (o_dt == FSK_F16) launch_reduce_out<D, kF16>(rp, B, many, s);
+  else if (o_dt == FSK_BF16) launch_reduce_out<D, kBF16>(rp, B, many, s);
+  else launch_reduce_out<D, kF32>(rp, B, many, s);
 }
 
 // The split policy's per-call constants (see SplitArgs): target_units <=
@@ -3396,10 +3457,9 @@ int run_decode(const Common& c) {
   rp.Hq = c.Hq; rp.Hkv = c.Hkv; rp.G = G;
   rp.blk_max = p.blk_max; rp.lens = p.lens_out; rp.scores = (uint8_t*)c.scores; rp.nblk = c.nblk;
   const Launch lr{c.stream, nullptr, ev[2]};
-  const bool rows4 = sp.chunk_min != sp.chunk_max && (int64_t)c.B >= 2 * (int64_t)sp.target_units;
-  if (c.D == 64) launch_reduce<64>(rp, c.B, c.o_dt, rows4, lr);
-  else if (c.D == 128) launch_reduce<128>(rp, c.B, c.o_dt, rows4, lr);
-  else launch_reduce<256>(rp, c.B, c.o_dt, rows4, lr);
+  if (c.D == 64) launch_reduce<64>(rp, c.B, c.o_dt, lr);
+  else if (c.D == 128) launch_reduce<128>(rp, c.B, c.o_dt, lr);
+  else launch_reduce<256>(rp, c.B, c.o_dt, lr);
   timing_keep(ev, true);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(FSK_ERR_HIP, std::string("kernel launch failed: ") + hipGetErrorString(e));

@@ -952,3 +952,22 @@ def test_concurrent_streams_and_threads_match_serial():
     torch.cuda.synchronize()
     assert all(torch.equal(o, want_a) for o in got[0])
     assert all(torch.equal(o, want_b) for o in got[1])
+
+
+# Batches of more than 2048 output rows: sequences of at most 16 partials merge
+# several rows per workgroup, longer ones (here of 17 and 47, over both blocks
+# of 256 sequences and more rows than the workgroups set aside for them) one.
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (64, 8, 64), (32, 8, 256), (36, 4, 128)])
+@pytest.mark.parametrize("mode", ["exp", "linear"])
+def test_many_rows_reduce(Hq, Hkv, D, mode):
+    lens = [(13 * b) % 97 for b in range(300)]
+    for b in range(0, 300, 13):
+        lens[b] = (512, 513, 1500)[b % 3]
+    wl = W.make("M0", overrides=dict(B=300, Hq=Hq, Hkv=Hkv, D=D, lens=("list", lens), sinks=True), seed=Hq + D)
+    # Sinks >= 0: the linear fold's denominator (the largest term, 1, plus the
+    # others and the sink) then is at least 1 and does not magnify P's rounding
+    # (2^-11 of each term) beyond the bar; with N(0, 1) sinks one of these 9600
+    # rows, of two tokens, has a sink near minus its sum.
+    wl.s_aux = wl.s_aux.abs()
+    run_and_check(wl, mode, chunk_tokens=32, what=f"{Hq}/{Hkv} D={D} {mode}, splits of 32")
+    run_and_check(wl, mode, what=f"{Hq}/{Hkv} D={D} {mode}")

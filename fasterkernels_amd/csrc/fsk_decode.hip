@@ -1,6 +1,6 @@
 // fsk_decode.hip -- split-KV GQA flash decoding for MI355X (gfx950).
 //
-// Two kernels per decode call:
+// Two kernels per decode call, or one for short sequences:
 //   1. partial_kernel: a persistent grid of one-wave workgroups walks a device
 //      work list of (sequence chunk, kv head) units (varlen at head_dim 64:
 //      a pair of neighbouring kv heads read as one 128-wide row).  Each unit streams its
@@ -16,7 +16,14 @@
 //      kernel arguments instead (HostPlan).
 //   2. reduce_kernel: one 256-thread workgroup per (sequence, query head) combines the
 //      partials with a log-sum-exp merge, folds the attention sink and writes
-//      the output in the requested dtype.
+//      the output in the requested dtype (reduce_many_kernel: several rows per
+//      workgroup for large batches).
+//   direct_kernel does all of it in one launch where every sequence that the
+//   call can hold is short: one workgroup per sequence and head, its waves
+//   merged through LDS.
+// Around them: the KV write, the e4m3 quantiser, the attended ranges of an HF
+// decode step, and the fp8 attention hook's decode, whose kernels (kinds kQuant
+// + type) quantise 16-bit K and V on the way to the matrix cores.
 //
 // The maths follows the reference kernels: scores s = q.k * sm_scale,
 // online softmax, P rounded to the KV compute type before P.V

@@ -439,7 +439,8 @@ FSK_API int fsk_set_option(const char *name, int64_t value);
  * process-wide, for one thread at a time).
  * With every_n > 0, every n-th decode or write call launches its kernels with
  * HIP events that the dispatches stamp (hipExtLaunchKernel): for a decode,
- * the split-KV partial kernel's start and end and the reduce kernel's end;
+ * the split-KV partial kernel's start and end and the reduce kernel's end (a
+ * direct call: its only kernel's start and end);
  * for a write, the write kernel's start and end.  every_n = 0 disables the
  * hook.  A timed launch costs ~20 us of extra host time, so time steps with
  * the hook off.  Not for use under HIP graph capture.  fsk_kernel_timing()

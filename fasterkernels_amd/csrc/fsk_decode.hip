@@ -3135,11 +3135,13 @@ void launch_reduce_out(const ReduceParams& rp, int B, bool many, const Launch& s
 }
 
 // More rows than workgroups fit at once (2048 of 256 threads on 256 CUs): see
-// reduce_many_kernel.
+// reduce_many_kernel.  Its grid is one-dimensional and a launch takes fewer than
+// 2^32 threads along a dimension: 2^24 workgroups, past which every row keeps a
+// workgroup of its own (up to 65536 heads x 16384 sequences are accepted).
 template <int D>
 void launch_reduce(const ReduceParams& rp, int B, int o_dt, const Launch& s) {
   const int64_t rows = (int64_t)rp.Hq * B;
-  const bool many = rows > 2048 && rows < ((int64_t)1 << 31) - 4096 && rp.Hq % kManyRows<D> == 0 && !rp.scores;
+  const bool many = rows > 2048 && rows / kManyRows<D> + kLongGroups < (1 << 24) && rp.Hq % kManyRows<D> == 0 && !rp.scores;
   if (o_dt == FSK_F16) launch_reduce_out<D, kF16>(rp, B, many, s);
   else if (o_dt == FSK_BF16) launch_reduce_out<D, kBF16>(rp, B, many, s);
   else launch_reduce_out<D, kF32>(rp, B, many, s);

@@ -784,11 +784,13 @@ __device__ __forceinline__ int find_seq(const int32_t* pre, int B, int u) {
 // item per SIMD, not two: one wave per SIMD streams more evenly.)
 
 // First head_dim element of k-step i for k-group g (the same for Q and K).
-template <bool kKvFp8>
+template <int kKV>
 __device__ __forceinline__ int qk_dim0(int i, int g) {
   // 16-bit KV: k-step i reads the 16-byte chunk 4i+g of a row.
-  // e4m3 KV: one 16-byte chunk (4(i/2)+g) covers k-steps i and i+1.
-  return kKvFp8 ? 16 * (4 * (i >> 1) + g) + 8 * (i & 1) : 8 * (4 * i + g);
+  // e4m3 KV: one 16-byte chunk (4(i/2)+g) covers k-steps i and i+1.  Rows
+  // quantised on the way take the same order, so that their scores are summed
+  // as those of stored codes are.
+  return kKV == kE4M3 || is_quant(kKV) ? 16 * (4 * (i >> 1) + g) + 8 * (i & 1) : 8 * (4 * i + g);
 }
 
 template <int D, int kKV>
@@ -943,7 +945,8 @@ __device__ __forceinline__ LaneGeo<D, kKV> lane_geo(const Params& p, int lane, i
   }
 #pragma unroll
   for (int i = 0; i < LG::kReads; ++i) {
-    lg.kread[i] = 16 * (c * TR::kChunks + ((4 * i + g) ^ k_swizzle<TR::kChunks>(c)));
+    const int chunk = TR::kFp8 ? 4 * i + g : qk_dim0<kKV>(i, g) / 8;
+    lg.kread[i] = 16 * (c * TR::kChunks + (chunk ^ k_swizzle<TR::kChunks>(c)));
     asm volatile("" : "+v"(lg.kread[i]));
   }
   return lg;
@@ -1477,7 +1480,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kWavesPerEu)
           p.q + (int64_t)un.b * p.q_sb + (int64_t)((un.kvh + hs) * p.G + (head_ok ? head : 0)) * p.q_sh;
 #pragma unroll
       for (int i = 0; i < kSteps; ++i) {
-        const int dk = qk_dim0<kKvFp8>(i, g);  // dim of the (paired) K row
+        const int dk = qk_dim0<kKV>(i, g);  // dim of the (paired) K row
         const int d0 = pair ? (dk & 63) : dk;  // dim of this column's query row
         const bool q_ok = head_ok && (!pair || (dk >> 6) == hs);
         // Every lane loads (padding heads read head 0's row, then zero it):
@@ -1994,7 +1997,7 @@ void direct_kernel(const int32_t* lens_arg, const int32_t* starts_arg, int B_arg
     const uint8_t* qrow = p.q + (int64_t)b * p.q_sb + (int64_t)((kvh + hs) * p.G + (head_ok ? head : 0)) * p.q_sh;
 #pragma unroll
     for (int i = 0; i < kSteps; ++i) {
-      const int dk = qk_dim0<kKvFp8>(i, g);
+      const int dk = qk_dim0<kKV>(i, g);
       const int d0 = pair ? (dk & 63) : dk;
       const bool q_ok = head_ok && (!pair || (dk >> 6) == hs);
       u32x4 x;
@@ -3324,8 +3327,10 @@ int run_decode(const Common& c) {
   const int n_hb = (G + 15) / 16;
   const int cus = device_cus();
   if (c.chunk % 32 != 0) return fail(FSK_ERR_INVALID, "chunk_tokens must be a multiple of 32");
+  // (A quantising decode is split as the decode of the stored codes is: with
+  // the order of qk_dim0 it gives that decode's result bit for bit.)
   const SplitPlan sp = plan_split(c.layout, c.B, plan_heads(c.layout, c.D, c.Hkv, G), c.kv_extent, c.page_size,
-                                  c.chunk, cus, elem_bytes(c.kv_dt));
+                                  c.chunk, cus, c.pre ? 1 : elem_bytes(c.kv_dt));
   const bool pair =
       g_opt.head_pairs && pair_shape(c.layout, c.D, c.Hkv, G) && !c.scores && c.k_sh == 64 && c.v_sh == 64;
   if (c.layout == FSK_LAYOUT_PAGED && sp.chunk_max > kChunkMax)

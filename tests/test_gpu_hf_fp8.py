@@ -6,6 +6,7 @@ import torch
 
 pytest.importorskip("transformers")
 
+from fasterkernels_amd import native as nat  # noqa: E402
 from fskernels.hip import decode as dec  # noqa: E402
 from fskernels.hip import hf as H  # noqa: E402
 from tests.test_gpu_decode import assert_close, f64  # noqa: E402
@@ -43,8 +44,9 @@ def check(q, k, v, mask, what, **kw):
     out, _ = H.custom_hf_decode_attention_forward_fp8(None, q, k, v, mask, scaling, **kw)
     want = steps(q, k, v, mask, scaling, **kw)
     assert out.dtype == want.dtype and out.shape == want.shape
-    # The same codes and scales: the sums' order differs, and with it P's
-    # rounding to f16 (2^-11 of values up to ~1.3) and the output's own.
+    # The same codes and scales; where one of the two takes the direct kernel
+    # the sums' order differs, and with it P's rounding to f16 (2^-11 of values
+    # up to ~1.3) and the output's own.
     ulp = 2.0 ** -7 if q.dtype == torch.bfloat16 else 2.0 ** -9
     assert_close(out, f64(want), 1e-3, ulp, what)
 
@@ -57,6 +59,23 @@ def test_matches_the_three_steps(S, D, dtype):
     q, k, v = inputs(3, 16, 4, S, D, dtype, seed=S + D)
     check(q, k, v, padding_mask(3, S, dtype), f"S={S} D={D} {dtype}")
     check(q, k, v, None, f"S={S} D={D} {dtype} no mask")
+
+
+# The split kernels quantising on the way give the very result of the stored
+# codes' decode: the split, the tiles and every sum's order are the same.
+@pytest.mark.parametrize("S,Hq,Hkv", [(1, 16, 4), (33, 16, 4), (700, 6, 2), (5000, 16, 4), (16000, 32, 2)])
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_split_results_are_those_of_the_stored_codes(S, Hq, Hkv, D, dtype):
+    q, k, v = inputs(3, Hq, Hkv, S, D, dtype, seed=S + D)
+    mask, scaling = padding_mask(3, S, dtype), 0.7 * D ** -0.5
+    nat.set_option("direct", 0)
+    try:
+        for m in (mask, None):
+            out, _ = H.custom_hf_decode_attention_forward_fp8(None, q, k, v, m, scaling)
+            assert torch.equal(out, steps(q, k, v, m, scaling)), f"S={S} D={D} {dtype} mask={m is not None}"
+    finally:
+        nat.set_option("direct", 1)
 
 
 @pytest.mark.parametrize("Hq,Hkv", [(8, 8), (64, 4), (3, 1), (40, 2)])

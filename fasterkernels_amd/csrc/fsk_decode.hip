@@ -3401,7 +3401,13 @@ int run_decode(const Common& c) {
     p.lens = nullptr;  // (host memory: the kernel takes the plan instead)
   }
 
-  if (c.pre) launch_pre(*c.pre, c.stream);
+  if (c.pre) {
+    // Its own check: the decode below clears the error state before its launches.
+    (void)hipGetLastError();
+    launch_pre(*c.pre, c.stream);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return fail(FSK_ERR_HIP, std::string("range and maxima kernel launch failed: ") + hipGetErrorString(e));
+  }
   if (const int waves = direct_waves(c, (int64_t)c.B * p.n_items_h)) {
     DirectParams dp;
     memset(&dp, 0, sizeof(dp));

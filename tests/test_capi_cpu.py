@@ -212,6 +212,27 @@ def test_varlen_and_dense_validation(lib):
     assert b"scale" in lib.fsk_last_error()
 
 
+def dense_fp8_args(**kw):
+    """A valid argument set for fsk_decode_dense_fp8 (fake pointers), overridable."""
+    a = dict(q=FAKE, q_sb=32 * 128, q_sh=128, q_n=4 * 32 * 128, k=FAKE, k_sb=8 * 512 * 128, k_sh=512 * 128, k_st=128,
+             k_n=4 * 8 * 512 * 128, v=FAKE, v_sb=8 * 512 * 128, v_sh=512 * 128, v_st=128, v_n=4 * 8 * 512 * 128, S=512,
+             mask=FAKE, mdt=nat.FSK_BF16, m_sb=512, m_ss=1, position=None, window=-1, out=FAKE, o_sb=32 * 128,
+             o_sh=128, B=4, Hq=32, Hkv=8, D=128, dt=nat.FSK_BF16, odt=nat.FSK_BF16, scale=0.088, ws=FAKE,
+             wsb=1 << 30, chunk=0, stream=None)
+    a.update(kw)
+    return list(a.values())
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="fake pointers: the launches have to fail")
+@pytest.mark.parametrize("S", [256, 512, 8192])
+def test_a_failed_first_launch_is_reported(lib, S):
+    """The quantising decode launches twice or three times: an error of the
+    first launch is returned, and the decode that would read what it had not
+    written is not launched."""
+    assert lib.fsk_decode_dense_fp8(*dense_fp8_args(S=S)) == nat.FSK_ERR_HIP
+    assert lib.fsk_last_error().startswith(b"range and maxima kernel launch failed")
+
+
 def test_debug_entry_validation(lib):
     assert lib.fsk_fp8_decode_table(None, None) == nat.FSK_ERR_INVALID
     assert lib.fsk_paged_gather(None, 0, 0, 0, FAKE, 4, 4, FAKE, 8, 16, 2, 8, 128, 0, FAKE, None) == nat.FSK_ERR_INVALID

@@ -80,14 +80,16 @@ void on_device(const at::Tensor& t, const char* name, const c10::Device& dev) {
     raise(kRuntime, std::string(name) + " is on " + t.device().str() + ", expected " + dev.str());
 }
 
-// The tensor itself when its innermost dim is contiguous and every row starts
-// 16-byte aligned (what the kernels' vector loads need), else a packed copy.
-at::Tensor rows16(const at::Tensor& t) {
+// Whether the innermost dim is contiguous and every row starts 16-byte aligned
+// (what the kernels' vector loads need).
+bool has_rows16(const at::Tensor& t) {
   const int64_t es = t.element_size();
   bool ok = t.stride(-1) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
   for (int64_t i = 0; ok && i + 1 < t.dim(); ++i) ok = (t.stride(i) * es) % 16 == 0;
-  return ok ? t : t.contiguous();
+  return ok;
 }
+// The tensor itself where it has such rows, else a packed copy.
+at::Tensor rows16(const at::Tensor& t) { return has_rows16(t) ? t : t.contiguous(); }
 
 at::Tensor int32_contig(const at::Tensor& t, const char* name, const c10::Device& dev) {
   on_device(t, name, dev);
@@ -524,7 +526,10 @@ at::Tensor dense_hf(const at::Tensor& q_in, const at::Tensor& k_cache, const at:
 
 // The fp8 attention hook's decode (triton_gqa_decode_hf_fp8.py:230-283): q
 // [B, Hq, 1, D] and k/v [>= B, Hkv, S, D] of one 16-bit type, quantised per
-// tensor on the way.  Tensors with gaps or unaligned rows are packed first.
+// tensor on the way.  Tensors with gaps, an unaligned start or rows, or a token
+// stride past the kernels' 32-bit offsets are copied first, as the codes' own
+// pass copies them (a contiguous one at an odd offset too: contiguous() would
+// return it as it is).
 at::Tensor dense_fp8(const at::Tensor& q_in, const at::Tensor& k_in, const at::Tensor& v_in,
                      const c10::optional<at::Tensor>& mask, const c10::optional<at::Tensor>& position,
                      c10::optional<int64_t> window, c10::optional<double> sm_scale, int64_t chunk_tokens,
@@ -534,8 +539,8 @@ at::Tensor dense_fp8(const at::Tensor& q_in, const at::Tensor& k_in, const at::T
   const c10::Device dev = q_in.device();
   const c10::DeviceGuard guard(dev);
   auto packed = [](const at::Tensor& t) {
-    const at::Tensor r = rows16(t);
-    return r.is_non_overlapping_and_dense() ? r : r.clone(at::MemoryFormat::Contiguous);
+    const bool ok = has_rows16(t) && t.is_non_overlapping_and_dense() && t.stride(-2) < (int64_t)1 << 26;
+    return ok ? t : t.clone(at::MemoryFormat::Contiguous);
   };
   on_device(k_in, "k_cache", dev);
   on_device(v_in, "v_cache", dev);

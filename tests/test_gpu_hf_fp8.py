@@ -99,12 +99,22 @@ def test_positions_windows_and_hints():
 
 
 def test_strides():
-    """Views with gaps, unaligned rows and permuted heads; a cache with more
-    sequences than the batch (its scales cover all of them)."""
+    """Views with gaps, permuted heads, contiguous tensors that do not start
+    16-byte aligned and rows of an odd stride; a cache with more sequences than
+    the batch (its scales cover all of them)."""
     q, k, v = inputs(4, 16, 4, 520, 128, torch.bfloat16)
     check(q, k[:, :, 3:400], v[:, :, 3:400], None, "gaps")
     check(q.transpose(0, 1).contiguous().transpose(0, 1), k.transpose(1, 2).contiguous().transpose(1, 2),
           v.transpose(1, 2).contiguous().transpose(1, 2), None, "permuted")
+    for at in range(3):
+        t = [q, k, v]
+        off = torch.empty(t[at].numel() + 8, dtype=q.dtype, device=DEV)
+        t[at] = off[3:3 + t[at].numel()].view(t[at].shape).copy_(t[at])
+        assert t[at].is_contiguous() and t[at].data_ptr() % 16
+        check(*t, None, f"tensor {at} at an odd offset")
+        wide = torch.empty(*[q, k, v][at].shape[:-1], 131, dtype=q.dtype, device=DEV)
+        t[at] = wide[..., :128].copy_([q, k, v][at])
+        check(*t, None, f"tensor {at} with rows of 131")
     k[3] *= 5
     check(q[:2], k, v, None, "more sequences than the batch")
     check(q, k[:1].expand(4, -1, -1, -1), v, None, "expanded")

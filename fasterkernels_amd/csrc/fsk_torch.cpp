@@ -529,7 +529,7 @@ at::Tensor dense_hf(const at::Tensor& q_in, const at::Tensor& k_cache, const at:
 // tensor on the way.  Tensors with gaps, an unaligned start or rows, or a token
 // stride past the kernels' 32-bit offsets are copied first, as the codes' own
 // pass copies them (a contiguous one at an odd offset too: contiguous() would
-// return it as it is).
+// return it as it is), and so are lazily negated ones.
 at::Tensor dense_fp8(const at::Tensor& q_in, const at::Tensor& k_in, const at::Tensor& v_in,
                      const c10::optional<at::Tensor>& mask, const c10::optional<at::Tensor>& position,
                      c10::optional<int64_t> window, c10::optional<double> sm_scale, int64_t chunk_tokens,
@@ -539,7 +539,7 @@ at::Tensor dense_fp8(const at::Tensor& q_in, const at::Tensor& k_in, const at::T
   const c10::Device dev = q_in.device();
   const c10::DeviceGuard guard(dev);
   auto packed = [](const at::Tensor& t) {
-    const bool ok = has_rows16(t) && t.is_non_overlapping_and_dense() && t.stride(-2) < (int64_t)1 << 26;
+    const bool ok = !t.is_neg() && has_rows16(t) && t.is_non_overlapping_and_dense() && t.stride(-2) < (int64_t)1 << 26;
     return ok ? t : t.clone(at::MemoryFormat::Contiguous);
   };
   on_device(k_in, "k_cache", dev);
@@ -567,7 +567,8 @@ at::Tensor dense_fp8(const at::Tensor& q_in, const at::Tensor& k_in, const at::T
 // e4m3 quantisation (fskernels/triton/triton_gqa_decode_hf_fp8.py:13-16)
 // ---------------------------------------------------------------------------
 // (codes, scale) of each of 1 to 3 tensors of one dtype, in two launches.  The
-// codes keep a dense tensor's strides; other tensors are packed first.  Each
+// codes keep a dense tensor's strides; other tensors, and lazily negated ones
+// (the kernels read memory as it is), are packed first.  Each
 // scale is a 0-dim fp32 device tensor.
 std::vector<std::pair<at::Tensor, at::Tensor>> quantize(const std::vector<at::Tensor>& xs, int64_t stream) {
   if (xs.empty() || xs.size() > 3) raise(FSK_ERR_INVALID, "quantize takes 1 to 3 tensors");
@@ -585,7 +586,7 @@ std::vector<std::pair<at::Tensor, at::Tensor>> quantize(const std::vector<at::Te
     const at::Tensor& x = xs[i];
     on_device(x, "x", dev);
     if (x.scalar_type() != xs[0].scalar_type()) raise(FSK_ERR_INVALID, "the tensors must have one dtype");
-    const bool dense = x.is_non_overlapping_and_dense() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
+    const bool dense = !x.is_neg() && x.is_non_overlapping_and_dense() && reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
     src.push_back(dense ? x : x.clone(at::MemoryFormat::Contiguous));
     const at::Tensor codes = at::empty_like(src.back(), src.back().options().dtype(at::kFloat8_e4m3fn));
     const at::Tensor sc = at::empty({}, x.options().dtype(at::kFloat));

@@ -50,14 +50,16 @@ def set_num_splits_fp8(n: int) -> None:
 
 def _kernel_quantizes(x) -> bool:
     """Whether quantize_to_fp8 may leave torch's operators: a plain fp32
-    tensor, and nothing active that records or transforms operators (it would
-    not see the kernels' launch)."""
+    tensor whose memory holds its values (not a lazily negated one), and nothing
+    active that records or transforms operators (it would not see the kernels'
+    launch)."""
     return (type(x) is torch.Tensor and x.is_cuda and x.dtype is torch.float32
             and not (x.requires_grad and torch.is_grad_enabled())
             and not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
             and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and not torch._C._functorch.is_functorch_wrapped_tensor(x) and forward_ad._current_level < 0
-            and x.layout is torch.strided and x.numel() > 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
+            and x.layout is torch.strided and not x.is_neg() and not x._is_zerotensor()
+            and x.numel() > 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 
 def quantize_to_fp8(x: torch.Tensor):

@@ -120,6 +120,15 @@ def test_strides():
     check(q, k[:1].expand(4, -1, -1, -1), v, None, "expanded")
 
 
+def test_lazily_negated_tensors():
+    """Their memory holds the values with the other sign: the call on views is
+    the call on the values."""
+    t = inputs(2, 8, 2, 300, 128, torch.float16)
+    want, _ = H.custom_hf_decode_attention_forward_fp8(None, -t[0], t[1], -t[2], None, 0.1)
+    got, _ = H.custom_hf_decode_attention_forward_fp8(None, torch._neg_view(t[0]), t[1], torch._neg_view(t[2]), None, 0.1)
+    assert torch.equal(got, want)
+
+
 # One special value in K, V or Q reaches every scale's codes as torch's max and
 # casts carry it: the same elements come out NaN.
 @pytest.mark.parametrize("which", [0, 1, 2])

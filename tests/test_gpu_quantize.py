@@ -74,6 +74,16 @@ def test_three_tensors_at_once_keep_their_own_scales():
         assert torch.equal(scale, ws) and torch.equal(codes.view(torch.uint8), want.view(torch.uint8))
 
 
+def test_lazily_negated_tensors():
+    """Their memory holds the values with the other sign."""
+    x = torch.randn(5003, device=DEV)
+    neg = torch._neg_view(x)
+    assert neg.is_neg()
+    check(dec.quantize_to_fp8(neg), -x, "quantize_to_fp8")
+    for t in (x, x.half(), x.bfloat16()):
+        check(dec.quantize_each_to_fp8(torch._neg_view(t))[0], -t.float(), f"quantize_each_to_fp8 {t.dtype}")
+
+
 def test_recorded_calls_keep_the_torch_expression():
     x = torch.randn(64, device=DEV, requires_grad=True)
     _, scale = dec.quantize_to_fp8(x)

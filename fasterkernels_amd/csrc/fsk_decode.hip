@@ -3305,6 +3305,7 @@ int dispatch_direct_layout(int layout, const DirectParams& dp, int waves, int q_
 int direct_waves(const Common& c, int64_t groups) {
   if (!g_opt.direct || c.chunk > 0 || g_opt.chunk_tokens > 0 || g_opt.qk_engine != 0) return 0;
   const int64_t extent = c.layout == FSK_LAYOUT_PAGED ? c.kv_extent * c.page_size : c.kv_extent;
+  if (c.chunk < 0 && -(int64_t)c.chunk < extent) return 0;  // the caller asked for several parts a sequence
   const int64_t row = 2 * (int64_t)c.D * elem_bytes(c.kv_dt);  // K/V bytes of a token and head
   const bool many = groups >= 128;
   const int64_t most_kb = c.D == 256 && c.kv_dt != FSK_E4M3 ? (many ? 384 : 64) : (many ? 512 : 192);

@@ -422,8 +422,9 @@ FSK_API int fsk_decode_dense_fp8(const void *q, int64_t q_stride_b, int64_t q_st
  *                         and 192 KB with fewer than 128 workgroups; less for
  *                         16-bit KV at head_dim 256) run one workgroup per
  *                         sequence and head, with no partials and no reduce
- *                         kernel; 0: always the split kernels.  (A fixed
- *                         chunk_tokens split always takes the split kernels.)
+ *                         kernel; 0: always the split kernels.  (A call's fixed
+ *                         split, or a chunk cap below its longest possible
+ *                         sequence, always takes the split kernels.)
  *   "qk_engine"           0 (default): QK and PV on the matrix cores (MFMA);
  *                         1: the VALU formulation of the tile, for A/B
  *                         measurement (f16 q and KV, head_dim 128, at most 4

@@ -23,15 +23,18 @@ def option():
     set_option("direct", 1)
 
 
-def launches(wl, **kw):
-    """Kernels of one call: 1 on the direct kernel, 2 on the split kernels
-    (a recorded direct call's events stop with its only kernel)."""
+def kernels(fn):
+    """(direct kernels, partial kernels) that a call launches."""
     from torch.profiler import ProfilerActivity, profile
     with profile(activities=[ProfilerActivity.CUDA]) as prof:
-        W.run(wl, **kw)
+        fn()
         torch.cuda.synchronize()
     names = [e.key for e in prof.key_averages()]
     return sum("direct_kernel" in n for n in names), sum("partial_kernel" in n for n in names)
+
+
+def launches(wl, **kw):
+    return kernels(lambda: W.run(wl, **kw))
 
 
 EDGES = [1, 31, 32, 33, 64, 65, 127, 129, 255, 257, 500, 512]
@@ -162,6 +165,32 @@ def test_rule(kv, B, longest, direct, option):
         assert torch.equal(host, W.run(wl))
     option("direct", 0)
     assert launches(wl) == (0, 1)
+
+
+# a split-count hint makes every full-length sequence split: chunks of at most
+# ceil(S / n) tokens, rounded up to 32, keep the split kernels where that is
+# less than S
+@pytest.mark.parametrize("S,splits,direct", [(384, 1, 1), (384, 2, 0), (384, 8, 0), (64, 2, 0), (33, 2, 0), (32, 8, 1)])
+def test_split_hints_keep_the_split_kernels(S, splits, direct):
+    g = torch.Generator().manual_seed(S)
+    q, k, v = (torch.randn(*s, generator=g).half() for s in ((2, 8, 128), (2, 2, S, 128), (2, 2, S, 128)))
+    lens = torch.tensor([S, S - 5], dtype=torch.int32, device=DEV)
+    args = q.to(DEV), k.to(DEV), v.to(DEV), lens
+    (q8, sq), (k8, sk), (v8, sv) = (W._quantize(t.float()) for t in (q, k, v))
+    args8 = (q8.to(DEV), k8.to(DEV), v8.to(DEV), lens, sq.to(DEV), sk.to(DEV), sv.to(DEV), torch.float16)
+    ref = O.decode_dense(f64(q), f64(k), f64(v), lens.cpu().numpy(), None)
+    dec.set_num_splits_fp8(splits)
+    try:
+        assert kernels(lambda: dec.flash_decode_gqa_hf_fp8(*args8)) == (direct, 1 - direct)
+    finally:
+        dec.set_num_splits_fp8(1)
+    assert kernels(lambda: dec.flash_decode_gqa_hf_dense_optimized(*args, num_splits=splits)) == (direct, 1 - direct)
+    dec.set_num_splits(splits)
+    try:
+        assert kernels(lambda: dec.flash_decode_gqa_hf_dense_optimized(*args)) == (direct, 1 - direct)
+        assert_close(dec.flash_decode_gqa_hf_dense_optimized(*args), ref, 2e-3, 2e-3, f"S={S} splits={splits}")
+    finally:
+        dec.set_num_splits(1)
 
 
 def test_captured_and_replayed():

@@ -3278,40 +3278,63 @@ int dispatch_direct_layout(int layout, const DirectParams& dp, int waves, int q_
 }
 
 // Waves of a direct call's workgroups, or 0: the split kernels.  `groups`
-// workgroups, one per (sequence, head slot).
+// workgroups, one per (sequence, head slot); `pair`: two KV heads each.
 //
 // A workgroup streams from one CU at ~57 GB/s of fp16 K/V (2 MB in 37 us, by 4
 // waves or 8), the split kernels from all of them after ~5 us more of plan,
-// partials and second launch.  The line is drawn on the longest sequence the
-// call can hold (the table's or cache's width; varlen: all rows), since the
-// lengths are on the device: 192 KB of a head's K/V and 768 tokens for any
-// call, 512 KB and 1024 tokens where at least 128 workgroups spread over the
-// CUs.  16-bit rows of head_dim 256, whose tiles are not pipelined, stop at
-// 64 KB and 384 KB.  Paged, 8 KV heads x 128, us a step, split -> direct: fp16
-// 1 x 64 tokens 10.2 -> 6.9 (host time), 1 x 384 9.3 -> 7.4, 64 x 256 17.9 ->
-// 13.7, 256 x 64 23.8 -> 14.1, 256 x 512 94.7 -> 83.8, 1024 x U[1,256] 131 ->
-// 91, 16 x 1024 17.4 -> 15.3, 256 x U[1,1024] 100.9 -> 90.4; past the lines 4 x
-// 512 9.5 -> 9.0 (4 KV heads of 16 query heads: 9.7 -> 9.9), 4 x 1024 10.5 ->
-// 13.1, 64 x U[1,2048] 51.6 -> 53.0.  e4m3: 1 x 768 9.6 -> 9.0, 16 x 1024 13.4
-// -> 11.3, 256 x U[1,1024] 59.1 -> 51.5; past them 4 x 1024 10.1 -> 10.6, 4 x
-// 2048 11.9 -> 15.7.  fp16 head_dim 256: 1 x 64 10.1 -> 7.1, 64 x 384 39.9 ->
-// 34.3; past them 4 x 256 11.3 -> 12.0, 16 x 512 19.4 -> 20.0.
+// partials and second launch.  The lengths are on the device, so the lines are
+// drawn on the longest sequence that the call can hold (the table's or cache's
+// width; varlen: all rows), for the mixes that are worst for this kernel: one
+// or four sequences of that length among ones of 16 tokens, and 16 tokens
+// throughout.  What the split kernels need for those grows with the workgroups
+// and with the query heads of each (rows to reduce): the lines move up with
+// groups x sqrt(query heads of a workgroup).  Measured at seven head shapes,
+// fp16 and e4m3, 64 to 4096 workgroups, extents of 128 to 1024 tokens and six
+// mixes (replayed graphs, split against direct): 33 % off in the mean, 9 of
+// 8088 points over by more than 3 %, none by 5 %.  One line at 512 KB and 128
+// workgroups for every mix and up to 4 waves everywhere had 383 such points, up
+// to 78 %.  us, split -> direct, 8 KV heads x 128 of fp16, 32 query heads: 1 x
+// 64 tokens 8.4 -> 4.5, 1 x 384 8.4 -> 6.9, 16 x 512 11.1 -> 8.9 (one of 512
+// among 15 of 16: 8.8 -> 7.6), 64 x 256 16.2 -> 12.4, 64 x 896 40.7 -> 36.4 (one:
+// 11.4 -> 10.6), 256 x 64 23.7 -> 12.9, 256 x U[1,1024] 98.6 -> 83.4; past the
+// lines 16 x 1024 15.7 -> 14.5 but one 8.9 -> 10.8.  e4m3: 1 x 768 8.7 -> 8.5, 32 x
+// 896 16.2 -> 11.6, 256 x 1024 111 -> 84.  head_dim 256 fp16, whose tiles are not
+// pipelined: 16 x 256 12.6 -> 11.4, past the line 16 x 384 one 10.5 -> 12.3.
+// Pairs read two heads' rows, and a quantising decode converts them and reads
+// its maxima first: both count 1.5 times (fp8 hook, 16 x 512, one: 17.5 us split,
+// 19.9 direct).
 //
-// Waves: one per two tiles, up to 8 in a few workgroups (1 x 512: 8.1 us with 4
-// waves, 7.8 with 8; 16 x 1024 e4m3 11.8 and 11.2) and 4 in many (64 x 512
-// fp16: 23.4 with 4, 26.1 with 8: fewer workgroups of 8 waves' stages fit a
-// CU); one per four tiles past 1024 workgroups (1024 x U[1,256]: 91.0 with 2,
-// 105.3 with 4; 1024 x 64: 48.6 with 1, 52.6 with 2).
-int direct_waves(const Common& c, int64_t groups) {
+// Waves: one per two tiles, up to 4, or 8 in a few workgroups and for e4m3 while
+// a CU has one (64 x 512 fp16: 23.4 us with 4, 26.1 with 8).  Past 1024 workgroups
+// one per four tiles, and where the chip's eight waves a CU hold a quarter of
+// the workgroups or less, at most 2 (16-token sequences behind a table of 1024,
+// 16 heads on 16 x 128 fp16, 4096 workgroups: split 20 us, 33 with 4, 19 with 2;
+// the split kernels take longer per workgroup with more query heads, and 8 KB
+// stages leave more of a CU: lines 2048 to 4608).
+struct DirectLine {
+  int level;        // from this many groups x sqrt(query heads) on
+  int tokens;       // longest extent
+  int kb, kb_d256;  // ... and its K/V of a head: 16-bit rows of head_dim 256 (kb_d256), others
+};
+constexpr DirectLine kDirectLines[] = {{1536, 1024, 512, 384}, {768, 1024, 448, 384}, {512, 1024, 384, 384},
+                                       {256, 896, 320, 256},   {128, 896, 256, 256},  {0, 768, 192, 64}};
+int direct_waves(const Common& c, int64_t groups, bool pair) {
   if (!g_opt.direct || c.chunk > 0 || g_opt.chunk_tokens > 0 || g_opt.qk_engine != 0) return 0;
   const int64_t extent = c.layout == FSK_LAYOUT_PAGED ? c.kv_extent * c.page_size : c.kv_extent;
   if (c.chunk < 0 && -(int64_t)c.chunk < extent) return 0;  // the caller asked for several parts a sequence
-  const int64_t row = 2 * (int64_t)c.D * elem_bytes(c.kv_dt);  // K/V bytes of a token and head
-  const bool many = groups >= 128;
-  const int64_t most_kb = c.D == 256 && c.kv_dt != FSK_E4M3 ? (many ? 384 : 64) : (many ? 512 : 192);
-  if (extent > (many ? kDirectTokens : 768) || extent * row > most_kb * 1024) return 0;
+  const bool e4m3 = c.kv_dt == FSK_E4M3;
+  const int heads = std::min(c.Hq / c.Hkv, 16);
+  const double level = groups < 128 ? 0. : (double)groups * std::sqrt((double)heads);
+  const DirectLine* line = kDirectLines;
+  while (level < line->level) ++line;
+  int64_t row = 2 * (int64_t)c.D * elem_bytes(c.kv_dt);  // K/V bytes of a token and head
+  if (pair || c.pre) row = row * 3 / 2;
+  if (extent > line->tokens || extent * row > (c.D == 256 && !e4m3 ? line->kb_d256 : line->kb) * 1024) return 0;
   const int64_t tiles = cdiv(extent, 32);
-  const int64_t most = groups <= (c.kv_dt == FSK_E4M3 ? 128 : 16) ? kDirectMaxWaves : 4;
+  const int64_t two = (heads >= 4 ? 3072 : 2048) * (e4m3 || c.D == 64 ? 3 : 2) / 2;
+  const int64_t most = groups <= 16 || (e4m3 && groups <= 256 && extent > 2 * groups) ? kDirectMaxWaves
+                       : groups >= two                                                ? 2
+                                                                                      : 4;
   int waves = 1;
   if (groups > 1024)
     while (2 * waves <= std::min(tiles / 4, most)) waves *= 2;
@@ -3409,7 +3432,7 @@ int run_decode(const Common& c) {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(FSK_ERR_HIP, std::string("range and maxima kernel launch failed: ") + hipGetErrorString(e));
   }
-  if (const int waves = direct_waves(c, (int64_t)c.B * p.n_items_h)) {
+  if (const int waves = direct_waves(c, (int64_t)c.B * p.n_items_h, pair)) {
     DirectParams dp;
     memset(&dp, 0, sizeof(dp));
     dp.p = p;

@@ -418,13 +418,14 @@ FSK_API int fsk_decode_dense_fp8(const void *q, int64_t q_stride_b, int64_t q_st
  *                         packed heads read KV heads 2i and 2i+1 as one
  *                         128-wide row; 0: one KV head per wave
  *   "direct"              1 (default): calls whose sequences are bounded to
- *                         1024 tokens and 512 KB of a head's K/V (768 tokens
- *                         and 192 KB with fewer than 128 workgroups; less for
- *                         16-bit KV at head_dim 256) run one workgroup per
- *                         sequence and head, with no partials and no reduce
- *                         kernel; 0: always the split kernels.  (A call's fixed
- *                         split, or a chunk cap below its longest possible
- *                         sequence, always takes the split kernels.)
+ *                         768 tokens and 192 KB of a head's K/V (with 128 or
+ *                         more workgroups up to 1024 tokens and 512 KB, by
+ *                         their number; less for 16-bit KV at head_dim 256)
+ *                         run one workgroup per sequence and head, with no
+ *                         partials and no reduce kernel; 0: always the split
+ *                         kernels.  (A call's fixed split, or a chunk cap below
+ *                         its longest possible sequence, always takes the
+ *                         split kernels.)
  *   "qk_engine"           0 (default): QK and PV on the matrix cores (MFMA);
  *                         1: the VALU formulation of the tile, for A/B
  *                         measurement (f16 q and KV, head_dim 128, at most 4

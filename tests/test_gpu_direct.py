@@ -47,9 +47,9 @@ EDGES = [1, 31, 32, 33, 64, 65, 127, 129, 255, 257, 500, 512]
 def test_short_sequences(layout, D, kv, longest):
     q = "f16" if kv == "f16" else "bf16"
     lens = [n for n in EDGES if n <= longest] + [longest] + [0] * 5
-    Hkv = 16 if D == 256 else 4  # (head_dim 256: at least 128 workgroups beyond 64 tokens)
+    Hkv = 16 if D == 256 else 4  # (head_dim 256: at least 128 workgroups beyond 64 tokens, 256 beyond 256)
     if layout == "C1" and longest > 64:
-        lens = [longest // 2 - 1, 0, 1, longest // 2] + [0] * 5  # (varlen: the call's rows are the bound)
+        lens = [longest // 2 - 1, 0, 1, longest // 2] + [0] * 12  # (varlen: the call's rows are the bound)
     wl = W.make(layout, overrides=dict(B=len(lens), Hq=4 * Hkv, Hkv=Hkv, D=D, kv=kv, q=q, out=q, lens=("list", lens),
                                        sinks=True), seed=D + longest)
     for mode in ("exp", "linear"):
@@ -57,9 +57,11 @@ def test_short_sequences(layout, D, kv, longest):
     assert launches(wl.to(DEV)) == (1, 0)
 
 
-# one, two and four waves in many workgroups, eight in few, the longest sequences
+# one, two and four waves in many workgroups, eight in few (e4m3: in up to 256),
+# the longest sequences
 @pytest.mark.parametrize("kv", ["f16", "e4m3"])
-@pytest.mark.parametrize("B,longest", [(300, 64), (300, 250), (300, 513), (40, 1024), (2, 250), (16, 1024)])
+@pytest.mark.parametrize("B,longest", [(300, 64), (300, 250), (300, 1024), (400, 600), (128, 896), (40, 640), (2, 250),
+                                       (2, 384), (16, 512)])
 def test_wave_counts(kv, B, longest):
     q = "f16" if kv == "f16" else "bf16"
     lens = [(37 * b) % (longest + 1) for b in range(B - 1)] + [longest]
@@ -145,18 +147,20 @@ def test_block_scores(layout, out, mode, option):
     assert torch.equal(scores == 0, want_scores == 0)
 
 
-# (batch, longest sequence, direct): the rule's lines for 8 KV heads x 128 of
-# fp16 (192 KB a head below 128 workgroups, 512 KB from there) and of e4m3
-# (768 and 1024 tokens)
-@pytest.mark.parametrize("kv,B,longest,direct", [
-    ("f16", 1, 384, 1), ("f16", 1, 385, 0), ("f16", 15, 384, 1), ("f16", 15, 1024, 0), ("f16", 16, 1024, 1),
-    ("f16", 16, 1025, 0), ("f16", 300, 100, 1), ("e4m3", 1, 768, 1), ("e4m3", 2, 769, 0), ("e4m3", 20, 1024, 1),
-    ("e4m3", 20, 1025, 0)])
-def test_rule(kv, B, longest, direct, option):
+# (query heads, batch, longest sequence, direct): both sides of the rule's lines
+# for 8 KV heads x 128: fp16 by K/V bytes of a head, e4m3 by tokens
+@pytest.mark.parametrize("kv,Hq,B,longest,direct", [
+    ("f16", 32, 1, 384, 1), ("f16", 32, 1, 385, 0), ("f16", 32, 15, 384, 1), ("f16", 32, 15, 1024, 0),
+    ("f16", 32, 16, 640, 1), ("f16", 32, 16, 641, 0), ("f16", 32, 32, 768, 1), ("f16", 32, 32, 769, 0),
+    ("f16", 32, 48, 896, 1), ("f16", 32, 48, 897, 0), ("f16", 32, 96, 1024, 1), ("f16", 32, 96, 1025, 0),
+    ("f16", 8, 16, 512, 1), ("f16", 8, 16, 513, 0), ("f16", 8, 192, 1024, 1), ("f16", 8, 191, 1024, 0),
+    ("f16", 32, 300, 100, 1), ("e4m3", 32, 1, 768, 1), ("e4m3", 32, 2, 769, 0), ("e4m3", 32, 20, 896, 1),
+    ("e4m3", 32, 20, 897, 0), ("e4m3", 32, 32, 1024, 1), ("e4m3", 32, 32, 1025, 0)])
+def test_rule(kv, Hq, B, longest, direct, option):
     lens = [(7 * b) % longest + 1 for b in range(B - 1)] + [longest]
     q = "f16" if kv == "f16" else "bf16"
-    wl = W.make("M0", overrides=dict(B=B, lens=("list", lens), kv=kv, q=q, out=q), seed=B)
-    run_and_check(wl, what=f"{kv} {B} x {longest}")
+    wl = W.make("M0", overrides=dict(B=B, Hq=Hq, lens=("list", lens), kv=kv, q=q, out=q), seed=B)
+    run_and_check(wl, what=f"{kv} Hq={Hq} {B} x {longest}")
     wl = wl.to(DEV)
     assert launches(wl) == (direct, 1 - direct)
     assert launches(wl, chunk_tokens=64) == (0, 1)  # a fixed split is the split kernels'

@@ -1692,9 +1692,9 @@ struct ReduceParams {
 
 constexpr int kReduceThreads = 256;
 
-// Rows h0 .. h0 + kRows - 1 (query heads) of sequence b.
+// Rows h0 .. h0 + kRows - 1 (query heads) of sequence b (tid: threadIdx.x).
 template <int D, int kOut, int kRows>
-__device__ __forceinline__ void reduce_rows(const ReduceParams& p, int h0, int b) {
+__device__ __forceinline__ void reduce_rows(const ReduceParams& p, int h0, int b, int tid) {
   // Thread t of row r = t / (256 / kRows) owns the float4 column d4 = t %
   // (D/4) of unit group grp; group grp merges units grp, grp + kGroups, ...
   // with an online LSE update, loading kPer units per round trip, and the
@@ -1707,7 +1707,6 @@ __device__ __forceinline__ void reduce_rows(const ReduceParams& p, int h0, int b
   __shared__ float s_m[kRows][kGroups];
   __shared__ float s_l[kRows][kGroups];
   __shared__ f32x4 s_acc[kRows][kGroups][kD4];
-  const int tid = threadIdx.x;
   const int row = tid / kRowThreads;
   const int d4 = (tid - row * kRowThreads) % kD4;
   const int grp = (tid - row * kRowThreads) / kD4;
@@ -1829,46 +1828,59 @@ __device__ __forceinline__ void reduce_rows(const ReduceParams& p, int h0, int b
 // One workgroup per (query head, sequence).
 template <int D, int kOut>
 __global__ __launch_bounds__(kReduceThreads) void reduce_kernel(ReduceParams p) {
-  reduce_rows<D, kOut, 1>(p, blockIdx.x, blockIdx.y);
+  reduce_rows<D, kOut, 1>(p, blockIdx.x, blockIdx.y, threadIdx.x);
 }
 
 // For many rows (more than the 2048 workgroups that fit the chip at once),
 // where starting a workgroup per row is what takes the time (~1 ns each: 16384
 // rows 15 us, and leaving most of them at once was slower still).  Workgroups
-// kLongGroups + i merge kManyRows rows of a sequence of few partials each; the
-// sequences of many partials among them keep a workgroup per row, dealt to
-// the first kLongGroups workgroups, which look them up in the plan (eight such
-// rows read through one CU: 64 sequences of 16 tokens and one of 32000, 44 us
-// instead of 28).  Step times before and after, fp16, us: 64 query heads on 4 KV
-// heads x 128, 128 x 300 tokens 31.0 -> 27.5, 65 x 2048 61.4 -> 55.2; 64 on 8 x
-// 64, 65 x 300 20.2 -> 16.1, 65 lognormal 90.9 -> 83.5; 32 on 8 x 128, 128 x 2048
-// 179.2 -> 165.6, varlen 199 x U[76,422] 50.4 -> 46.9, one sequence of 32000
-// among 64 of 16 34.4 -> 32.0.  At 512 to 2048 rows the two differ by -3 to +5 %
+// kLongGroups + i merge kManyRows rows of a sequence of few partials each: 8
+// where the query heads divide by 8 and a row has at least two groups of
+// threads (head_dim up to 128), else 4.  The sequences of many partials among
+// them keep a workgroup per row, dealt to the first kLongGroups workgroups, which
+// look them up in the plan (eight such rows read through one CU: 64 sequences of
+// 16 tokens and one of 32000, 44 us instead of 28).  Step times with a workgroup
+// per row and so, fp16, us: 64 query heads on 4 KV heads x 128, 128 x 300 tokens
+// 30.5 -> 25.2, 65 x 2048 63.4 -> 56.5; 64 on 8 x 64, 65 x 300 19.9 -> 15.6, 65
+// lognormal 124.0 -> 115.4; 32 on 8 x 128, 128 x 2048 189.2 -> 175.1, one sequence
+// of 32000 among 64 of 16 32.9 -> 31.6; four rows a workgroup: 28 on 4 x 128, 512 x
+// 64 36.4 -> 31.5, 36 on 4 x 64, 512 x 300 56.8 -> 49.5, 12 on 4 x 256, one of 32000
+// among 511 of 16 61.4 -> 53.7.  At 512 to 2048 rows the two differ by -3 to +5 %
 // either way (64 lognormal 142.6 and 142.9), so one workgroup per row stays.
-template <int D>
-constexpr int kManyRows = D <= 128 ? 8 : 4;
+// kLongGroups = 512 took up to 3 us longer (28 on 4 x 128, 128 x U[1,1024] behind a
+// wide table: 32.1, with 256 29.2, with 128 29.0).
 constexpr int kFewUnits = 16;    // partials of a sequence that count as few
-constexpr int kLongGroups = 512;
-template <int D, int kOut>
+constexpr int kLongGroups = 256;
+template <int D, int kOut, int kManyRows>
 __global__ __launch_bounds__(kReduceThreads) void reduce_many_kernel(ReduceParams p, int B, FastDiv per_seq) {
   if ((int)blockIdx.x >= kLongGroups) {
     const uint32_t i = blockIdx.x - kLongGroups;
     const uint32_t b = fdiv(i, per_seq);  // per_seq = Hq / kManyRows workgroups of a sequence
     if (p.plan[b + 1] - p.plan[b] > kFewUnits) return;
-    reduce_rows<D, kOut, kManyRows<D>>(p, (int)(i - b * per_seq.d) * kManyRows<D>, (int)b);
+    reduce_rows<D, kOut, kManyRows>(p, (int)(i - b * per_seq.d) * kManyRows, (int)b, threadIdx.x);
     return;
   }
-  __shared__ uint64_t s_long[kReduceThreads / kWave];  // the long ones of kReduceThreads sequences
+  constexpr int kPasses = 4;  // of kReduceThreads sequences, in one round trip
+  constexpr int kMasks = kPasses * kReduceThreads / kWave;
+  __shared__ uint64_t s_long[kMasks];  // the long ones of them
   int row = blockIdx.x;  // of the long sequences' rows, in order; then every kLongGroups-th
   int before = 0;        // long sequences passed
-  for (int b0 = 0; b0 < B; b0 += kReduceThreads) {
-    const int b = b0 + (int)threadIdx.x;
-    const uint64_t is_long = __ballot(b < B && p.plan[min(b, B - 1) + 1] - p.plan[min(b, B - 1)] > kFewUnits);
-    if ((threadIdx.x & (kWave - 1)) == 0) s_long[threadIdx.x / kWave] = is_long;
+  for (int b0 = 0; b0 < B; b0 += kPasses * kReduceThreads) {
+    int n[kPasses];
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) {
+      const int b = min(b0 + i * kReduceThreads + (int)threadIdx.x, B - 1);
+      n[i] = p.plan[b + 1] - p.plan[b];
+    }
+#pragma unroll
+    for (int i = 0; i < kPasses; ++i) {
+      const uint64_t is_long = __ballot(b0 + i * kReduceThreads + (int)threadIdx.x < B && n[i] > kFewUnits);
+      if ((threadIdx.x & (kWave - 1)) == 0) s_long[(i * kReduceThreads + threadIdx.x) / kWave] = is_long;
+    }
     __syncthreads();
     int here = 0;
 #pragma unroll
-    for (int w = 0; w < kReduceThreads / kWave; ++w) here += __builtin_popcountll(s_long[w]);
+    for (int w = 0; w < kMasks; ++w) here += __builtin_popcountll(s_long[w]);
     here = uniform(here);
     for (int k = row / p.Hq; k < before + here; row += kLongGroups, k = row / p.Hq) {
       int left = k - before, w = 0;  // the left-th set bit of s_long
@@ -1879,7 +1891,11 @@ __global__ __launch_bounds__(kReduceThreads) void reduce_many_kernel(ReduceParam
       }
       while (left-- > 0) m &= m - 1;
       const int seq = uniform(b0 + w * kWave + __builtin_ctzll(m));
-      reduce_rows<D, kOut, 1>(p, row - k * p.Hq, seq);
+      // (what depends on the thread is worked out per row: kept over the loop
+      // it took 94 registers, with which five workgroups fit a CU, not seven)
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      reduce_rows<D, kOut, 1>(p, row - k * p.Hq, seq, tid);
       __syncthreads();
     }
     before += here;
@@ -3129,25 +3145,36 @@ FastDiv make_fastdiv(uint32_t d) {
 }
 
 template <int D, int kOut>
-void launch_reduce_out(const ReduceParams& rp, int B, bool many, const Launch& s) {
-  if (many)
-    launch(reduce_many_kernel<D, kOut>, dim3((unsigned)(kLongGroups + (int64_t)rp.Hq / kManyRows<D> * B)),
-           dim3(kReduceThreads), 0, s, rp, B, make_fastdiv((uint32_t)(rp.Hq / kManyRows<D>)));
-  else
+void launch_reduce_out(const ReduceParams& rp, int B, int rows, const Launch& s) {
+  if (rows == 1) {
     launch(reduce_kernel<D, kOut>, dim3(rp.Hq, B), dim3(kReduceThreads), 0, s, rp);
+    return;
+  }
+  const dim3 grid((unsigned)(kLongGroups + (int64_t)rp.Hq / rows * B));
+  const FastDiv per_seq = make_fastdiv((uint32_t)(rp.Hq / rows));
+  if constexpr (D <= 128) {
+    if (rows == 8) {
+      launch(reduce_many_kernel<D, kOut, 8>, grid, dim3(kReduceThreads), 0, s, rp, B, per_seq);
+      return;
+    }
+  }
+  launch(reduce_many_kernel<D, kOut, 4>, grid, dim3(kReduceThreads), 0, s, rp, B, per_seq);
 }
 
 // More rows than workgroups fit at once (2048 of 256 threads on 256 CUs): see
-// reduce_many_kernel.  Its grid is one-dimensional and a launch takes fewer than
-// 2^32 threads along a dimension: 2^24 workgroups, past which every row keeps a
-// workgroup of its own (up to 65536 heads x 16384 sequences are accepted).
+// reduce_many_kernel, with 8 rows a workgroup where the query heads divide by 8
+// (head_dim 256: by 4, with 4), else 4 where they divide by 4.  Its grid is
+// one-dimensional and a launch takes fewer than 2^32 threads along a dimension:
+// 2^24 workgroups, past which every row keeps a workgroup of its own (up to
+// 65536 heads x 16384 sequences are accepted).
 template <int D>
 void launch_reduce(const ReduceParams& rp, int B, int o_dt, const Launch& s) {
-  const int64_t rows = (int64_t)rp.Hq * B;
-  const bool many = rows > 2048 && rows / kManyRows<D> + kLongGroups < (1 << 24) && rp.Hq % kManyRows<D> == 0 && !rp.scores;
-  if (o_dt == FSK_F16) launch_reduce_out<D, kF16>(rp, B, many, s);
-  else if (o_dt == FSK_BF16) launch_reduce_out<D, kBF16>(rp, B, many, s);
-  else launch_reduce_out<D, kF32>(rp, B, many, s);
+  const int64_t total = (int64_t)rp.Hq * B;
+  int rows = D <= 128 && rp.Hq % 8 == 0 ? 8 : rp.Hq % 4 == 0 ? 4 : 1;
+  if (total <= 2048 || total / rows + kLongGroups >= (1 << 24) || rp.scores) rows = 1;
+  if (o_dt == FSK_F16) launch_reduce_out<D, kF16>(rp, B, rows, s);
+  else if (o_dt == FSK_BF16) launch_reduce_out<D, kBF16>(rp, B, rows, s);
+  else launch_reduce_out<D, kF32>(rp, B, rows, s);
 }
 
 // The split policy's per-call constants (see SplitArgs): target_units <=

@@ -955,15 +955,17 @@ def test_concurrent_streams_and_threads_match_serial():
 
 
 # Batches of more than 2048 output rows: sequences of at most 16 partials merge
-# several rows per workgroup, longer ones (here of 17 and 47, over both blocks
-# of 256 sequences and more rows than the workgroups set aside for them) one.
-@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (64, 8, 64), (32, 8, 256), (36, 4, 128)])
+# several rows per workgroup (four where the query heads do not divide by 8),
+# longer ones (here of 17 and 47, over all passes of 256 sequences and both
+# rounds of 1024, and more rows than the workgroups set aside for them) one.
+@pytest.mark.parametrize("Hq,Hkv,D,B", [(32, 8, 128, 300), (64, 8, 64, 300), (32, 8, 256, 300), (36, 4, 128, 300),
+                                        (36, 4, 64, 300), (12, 4, 256, 300), (12, 2, 128, 1100), (9, 3, 128, 300)])
 @pytest.mark.parametrize("mode", ["exp", "linear"])
-def test_many_rows_reduce(Hq, Hkv, D, mode):
-    lens = [(13 * b) % 97 for b in range(300)]
-    for b in range(0, 300, 13):
+def test_many_rows_reduce(Hq, Hkv, D, B, mode):
+    lens = [(13 * b) % 97 for b in range(B)]
+    for b in range(0, B, 13):
         lens[b] = (512, 513, 1500)[b % 3]
-    wl = W.make("M0", overrides=dict(B=300, Hq=Hq, Hkv=Hkv, D=D, lens=("list", lens), sinks=True), seed=Hq + D)
+    wl = W.make("M0", overrides=dict(B=B, Hq=Hq, Hkv=Hkv, D=D, lens=("list", lens), sinks=True), seed=Hq + D)
     # Sinks >= 0: the linear fold's denominator (the largest term, 1, plus the
     # others and the sink) then is at least 1 and does not magnify P's rounding
     # (2^-11 of each term) beyond the bar; with N(0, 1) sinks one of these 9600
@@ -971,3 +973,21 @@ def test_many_rows_reduce(Hq, Hkv, D, mode):
     wl.s_aux = wl.s_aux.abs()
     run_and_check(wl, mode, chunk_tokens=32, what=f"{Hq}/{Hkv} D={D} {mode}, splits of 32")
     run_and_check(wl, mode, what=f"{Hq}/{Hkv} D={D} {mode}")
+
+
+# One row a workgroup up to 2048 rows and for query heads that do not divide by
+# 4; else eight (head_dim 256: four), or four where they do not divide by 8.
+@pytest.mark.parametrize("Hq,D,B,kernel", [
+    (8, 128, 256, "reduce_kernel<128, 0>"), (8, 128, 257, "reduce_many_kernel<128, 0, 8>"),
+    (4, 128, 513, "reduce_many_kernel<128, 0, 4>"), (12, 64, 171, "reduce_many_kernel<64, 0, 4>"),
+    (8, 256, 257, "reduce_many_kernel<256, 0, 4>"), (6, 128, 600, "reduce_kernel<128, 0>")])
+def test_rows_of_a_reduce_workgroup(Hq, D, B, kernel):
+    from torch.profiler import ProfilerActivity, profile
+    wl = W.make("M0", overrides=dict(B=B, Hq=Hq, Hkv=2, D=D, lens=("list", [1 + b % 40 for b in range(B)]),
+                                     max_blocks=128), seed=B)
+    run_and_check(wl, what=kernel)
+    wl = wl.to(DEV)
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        W.run(wl)
+        torch.cuda.synchronize()
+    assert any(kernel in e.key for e in prof.key_averages()), [e.key for e in prof.key_averages()]

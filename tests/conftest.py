@@ -20,3 +20,13 @@ def pytest_collection_modifyitems(config, items):
     for item in items:
         if "gpu" in item.keywords:
             item.add_marker(skip)
+
+
+@pytest.fixture(params=["direct", "split"])
+def both_routes(request):
+    """Calls of short sequences as they are routed, on the direct kernel, and
+    again with every call on the split kernels."""
+    from fasterkernels_amd import native as nat
+    nat.set_option("direct", int(request.param == "direct"))
+    yield
+    nat.set_option("direct", 1)

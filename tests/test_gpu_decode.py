@@ -158,6 +158,7 @@ def test_paged_reference_case(kv):
         assert_close(out, oracle_for(wl), 1e-3, 1e-3, f"paged {kv} at 1e-3", bare=True)
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("lens", [[1], [15], [16], [17], [31], [32], [33], [1, 2, 3, 4, 5, 6, 7],
                                   [0, 5, 0, 40]])
 def test_paged_edge_lengths(lens):
@@ -240,6 +241,7 @@ def test_varlen_large_groups_with_sinks(Hq, Hkv):
     run_and_check(wl, what=f"varlen G={Hq // Hkv}")
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("D", [64, 256])
 @pytest.mark.parametrize("kv", ["f16", "bf16", "e4m3"])
 def test_paged_head_dims(D, kv):
@@ -323,6 +325,7 @@ def test_varlen_reference_case(mode):
     assert_close(out, oracle_for(wl, mode), 1e-3, 1e-3, f"varlen ref {mode} at 1e-3", bare=True)
 
 
+@pytest.mark.usefixtures("both_routes")
 def test_varlen_zero_and_tiny():
     wl = W.make("C1", overrides=dict(B=6, lens=("list", [0, 1, 2, 0, 33, 3]), sinks=True), seed=4)
     run_and_check(wl, what="varlen tiny + sinks")
@@ -664,6 +667,7 @@ def test_hip_graph_replays_match_eager():
         assert torch.equal(static_out, eager), f"replay {i} differs from the eager result"
 
 
+@pytest.mark.usefixtures("both_routes")
 def test_zero_length_with_very_negative_sink():
     """An empty sequence with a sink far below zero: output 0, not NaN."""
     wl = W.make("C1", overrides=dict(B=3, lens=("list", [0, 5, 0]), sinks=True), seed=35)
@@ -671,6 +675,7 @@ def test_zero_length_with_very_negative_sink():
     run_and_check(wl, what="empty + sink -200")
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("sinks", [False, True])
 def test_all_empty_varlen_batch(sinks):
     """Every sequence empty and K/V with zero rows (null data pointers): the
@@ -692,6 +697,7 @@ def _lens(B, hi, seed):
     return lens
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("layout", ["varlen", "paged"])
 def test_batches_above_one_wave(layout):
     name = "C1" if layout == "varlen" else "C3"
@@ -701,6 +707,7 @@ def test_batches_above_one_wave(layout):
     run_and_check(wl, chunk_tokens=64, what=f"{layout} B=150 chunk 64")
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("B", [63, 64, 65])
 @pytest.mark.parametrize("layout", ["varlen", "paged"])
 def test_batches_at_one_wave_with_empty_runs(layout, B):
@@ -718,12 +725,13 @@ def test_batches_at_one_wave_with_empty_runs(layout, B):
     run_and_check(wl, chunk_tokens=32, what=f"{layout} B={B} chunk 32")
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("mode", ["exp", "linear"])
 def test_large_batch_reduce_rows(D, mode):
-    """Batches of at least twice as many sequences as the split has chunks
-    merge four query heads per reduce workgroup: 300 short sequences (some
-    empty), sinks in both folds, every head dim."""
+    """300 short sequences (some empty), 9600 output rows, sinks in both folds,
+    every head dim: the split kernels' reduce merges several query heads per
+    workgroup."""
     r = np.random.default_rng(D)
     lens = [int(x) for x in r.integers(0, 400, 300)]
     wl = W.make("C3", overrides=dict(B=300, D=D, lens=("list", lens), sinks=True), seed=D)
@@ -732,6 +740,7 @@ def test_large_batch_reduce_rows(D, mode):
     run_and_check(wl, sink_mode=mode, what=f"B=300 D={D} {mode}")
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("chunk", [0, 32, 64, 128])
 def test_paged_large_batch_row_ends(chunk):
     """Paged batches over 64 sequences load each segment's length together
@@ -746,6 +755,7 @@ def test_paged_large_batch_row_ends(chunk):
     run_and_check(wl, chunk_tokens=chunk, what=f"B=100 max_blocks=33 chunk={chunk}")
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("layout", ["varlen", "paged"])
 def test_maximum_batch(layout):
     """The largest batch the library takes (16384 sequences): the plan keeps
@@ -758,6 +768,7 @@ def test_maximum_batch(layout):
     run_and_check(wl, what=f"{layout} B={B}")
 
 
+@pytest.mark.usefixtures("both_routes")
 def test_dense_batch_above_one_wave():
     B = 70
     lens = _lens(B, 300, 53)
@@ -882,6 +893,7 @@ def test_randomized_large_batches(seed):
     run_and_check(wl, chunk_tokens=chunk, what=f"seed {seed}: {name} B={ov['B']} chunk={chunk}")
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("seed", range(20))
 def test_randomized_dense_configurations(seed):
     """Dense HF-cache layout: random batch, cache size, lengths, start offsets,

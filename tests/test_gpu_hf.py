@@ -58,6 +58,7 @@ def mask_from_ranges(B, S, starts, ends):
     return torch.where(ok, 0.0, NEG)[:, None, None, :].to(DEV)
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("name,starts,ends", [
     ("dynamic cache", [0, 0, 0], [300, 300, 300]),
     ("left padding", [0, 37, 299], [300, 300, 300]),

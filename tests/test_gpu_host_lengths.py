@@ -62,6 +62,7 @@ CASES = [
 ]
 
 
+@pytest.mark.usefixtures("both_routes")
 @pytest.mark.parametrize("name,ov,mode,chunk", CASES)
 def test_host_lengths_bit_identical(name, ov, mode, chunk):
     wl = W.make(name, overrides=ov, seed=21).to(DEV)
@@ -109,6 +110,7 @@ def test_host_lengths_64_sequences():
         assert_same(d, h, f"C5 {mode}")
 
 
+@pytest.mark.usefixtures("both_routes")
 def test_host_lengths_beyond_64_sequences_use_device_copy():
     """More than 64 sequences: the binding copies the host lengths to the
     device and takes the device-plan path, with the same result."""
@@ -125,6 +127,7 @@ def test_host_lengths_with_block_scores_use_device_copy(layout):
     assert_same(d, h, f"{layout} with block scores")
 
 
+@pytest.mark.usefixtures("both_routes")
 def test_host_lengths_clamped_like_device_ones():
     """Out-of-range lengths are clamped the same way on both paths: paged
     lengths to [0, max_blocks * page_size], varlen offsets to [0, T] and

@@ -3878,6 +3878,9 @@ int64_t fsk_workspace_bytes(int layout, int batch, int num_q_heads, int num_kv_h
   if (head_dim != 64 && head_dim != 128 && head_dim != 256) return fail(FSK_ERR_UNSUPPORTED, "head_dim must be 64, 128 or 256");
   if (layout == FSK_LAYOUT_PAGED && (page_size <= 0 || page_size % 16)) return fail(FSK_ERR_UNSUPPORTED, "page_size must be a positive multiple of 16");
   if (chunk_tokens % 32) return fail(FSK_ERR_INVALID, "chunk_tokens: a multiple of 32");
+  // (no decode takes them, and the products below would leave int64)
+  if (kv_extent >= ((int64_t)1 << 31) || (layout == FSK_LAYOUT_PAGED && kv_extent * page_size >= ((int64_t)1 << 31)))
+    return fail(FSK_ERR_UNSUPPORTED, "kv extent out of int32 range");
   const int G = num_q_heads / num_kv_heads;
   const int B = batch > 0 ? batch : 1;
   // sized for 16-bit KV: the smallest chunk_pref, so the most chunks

@@ -101,6 +101,13 @@ def test_workspace_sizes_reject_overflowing_shapes(lib):
     assert lib.fsk_score_workspace_bytes(16384, 1 << 16, 1 << 24) > 0
     assert lib.fsk_workspace_bytes(nat.FSK_LAYOUT_PAGED, 4, 1 << 20, 8, 128, 2048, 16, 0) == nat.FSK_ERR_UNSUPPORTED
     assert lib.fsk_workspace_bytes(nat.FSK_LAYOUT_PAGED, 1 << 20, 32, 8, 128, 2048, 16, 0) == nat.FSK_ERR_UNSUPPORTED
+    # token extents that no decode takes
+    for layout, extent, page in ((nat.FSK_LAYOUT_DENSE, (1 << 63) - 1, 16), (nat.FSK_LAYOUT_VARLEN, 1 << 31, 16),
+                                 (nat.FSK_LAYOUT_PAGED, 1 << 62, 16), (nat.FSK_LAYOUT_PAGED, 1 << 27, 16),
+                                 (nat.FSK_LAYOUT_PAGED, 1 << 30, 1 << 30)):
+        assert lib.fsk_workspace_bytes(layout, 4, 32, 8, 128, extent, page, 0) == nat.FSK_ERR_UNSUPPORTED
+    for layout, extent in ((nat.FSK_LAYOUT_DENSE, (1 << 31) - 1), (nat.FSK_LAYOUT_PAGED, (1 << 27) - 1)):
+        assert lib.fsk_workspace_bytes(layout, 4, 32, 8, 128, extent, 16, 0) > 0
 
 
 def test_workspace_size_cache_is_bounded(lib, monkeypatch):

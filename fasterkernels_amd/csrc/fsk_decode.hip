@@ -3730,8 +3730,10 @@ int64_t quant_ws_bytes(int B) { return align256(3 * kAmaxMax * 4) + align256(8 *
 int run_quant_decode(const QuantDecode& a, Common c) {
   if (c.q_dt != c.kv_dt || (c.q_dt != FSK_F16 && c.q_dt != FSK_BF16))
     return fail(FSK_ERR_UNSUPPORTED, "q, k and v must be f16 or bf16, of one type");
-  if (c.Hkv > 0 && c.Hq > 16 * c.Hkv) return fail(FSK_ERR_UNSUPPORTED, "more than 16 query heads per KV head");
-  const int64_t own = quant_ws_bytes(std::max(c.B, 0));
+  if (c.B < 0 || c.Hq <= 0 || c.Hkv <= 0) return fail(FSK_ERR_INVALID, "batch/heads must be positive");
+  if (c.Hq > 16 * (int64_t)c.Hkv) return fail(FSK_ERR_UNSUPPORTED, "more than 16 query heads per KV head");
+  if (c.B > kMaxBatch) return fail(FSK_ERR_UNSUPPORTED, "batch above 16384");
+  const int64_t own = quant_ws_bytes(c.B);
   if (!c.ws || c.ws_bytes < own || !aligned(c.ws, 256))
     return fail(FSK_ERR_WORKSPACE, "workspace missing, unaligned or smaller than fsk_decode_dense_fp8_workspace_bytes()");
   uint8_t* ws = (uint8_t*)c.ws;

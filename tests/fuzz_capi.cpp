@@ -85,7 +85,20 @@ int main() {
                           pick_i64(), pick_i(), pick_i(), pick_i(), pick_i(), pick_i() & 3, pick_i() & 3,
                           (const float*)pick_p(), (const float*)pick_p(), (int32_t*)pick_p(), pick_i64(),
                           (const int64_t*)pick_p(), pick_i64(), nullptr), "write");
+    check(fsk_decode_bounds(pick_p(), (int)(rng() % 7) - 1, pick_i64(), pick_i64(), (const int64_t*)pick_p(),
+                            pick_i64(), pick_i(), pick_i(), (int32_t*)pick_p(), (int32_t*)pick_p(), nullptr), "bounds");
+    {
+      const void* src[3] = {pick_p(), pick_p(), pick_p()};
+      void* dst[3] = {pick_p(), pick_p(), pick_p()};
+      float* scale[3] = {(float*)pick_p(), (float*)pick_p(), (float*)pick_p()};
+      const int64_t numel[3] = {pick_i64(), pick_i64(), pick_i64()};
+      check(fsk_quantize_e4m3((int)(rng() % 6) - 1, rng() % 8 ? src : nullptr, rng() % 8 ? numel : nullptr,
+                              (int)(rng() % 6) - 1, rng() % 8 ? dst : nullptr, rng() % 8 ? scale : nullptr, pick_p(),
+                              pick_i64(), nullptr), "quantize");
+      (void)fsk_quantize_workspace_bytes(pick_i());
+    }
     check(fsk_set_option(rng() % 2 ? "xcd_skew" : "nope", pick_i64()), "set_option");
+    check(fsk_set_option("direct", (int64_t)(rng() % 4) - 1), "set_option direct");
   }
   // Valid paged arguments with 1-3 fields perturbed (deeper validation paths).
   for (int it = 0; it < 200000; ++it) {
@@ -115,6 +128,26 @@ int main() {
     (void)fsk_workspace_bytes((int)(rng() % 4), (int)a[24], (int)a[25], (int)a[26], (int)a[27], (a[13] & 0xFFFFFF) * 16,
                               (int)a[16], (int)a[34]);
   }
+  // Valid quantising-decode arguments with 1-3 fields perturbed.
+  for (int it = 0; it < 100000; ++it) {
+    int64_t a[34] = {0x100000, 32 * 128, 128, 4 * 32 * 128, 0x200000, 8 * 512 * 128, 512 * 128, 128, 4 * 8 * 512 * 128,
+                     0x300000, 8 * 512 * 128, 512 * 128, 128, 4 * 8 * 512 * 128, 512, 0x400000, 1, 512, 1, 0, -1,
+                     0x500000, 32 * 128, 128, 4, 32, 8, 128, 1, 1, 0, 0x700000, (int64_t)1 << 30, 0};
+    if (rng() % 2) a[15] = 0;  // without a mask
+    const int nper = 1 + rng() % 3;
+    for (int j = 0; j < nper; ++j) {
+      const int f = rng() % 34;
+      if (f == 30) continue;  // sm_scale slot (float)
+      a[f] = (f == 0 || f == 4 || f == 9 || f == 15 || f == 19 || f == 21 || f == 31) ? (int64_t)(uintptr_t)pick_p()
+                                                                                        : pick_i64();
+    }
+    check(fsk_decode_dense_fp8((void*)a[0], a[1], a[2], a[3], (void*)a[4], a[5], a[6], a[7], a[8], (void*)a[9], a[10],
+                               a[11], a[12], a[13], a[14], (void*)a[15], (int)a[16], a[17], a[18], (const int64_t*)a[19],
+                               a[20], (void*)a[21], a[22], a[23], (int)a[24], (int)a[25], (int)a[26], (int)a[27],
+                               (int)a[28], (int)a[29], 0.088f, (void*)a[31], a[32], (int)a[33], nullptr),
+          "dense-fp8-perturbed");
+    (void)fsk_decode_dense_fp8_workspace_bytes((int)a[24], (int)a[25], (int)a[26], (int)a[27], a[14], (int)a[33]);
+  }
   // Valid write arguments with 1-3 fields perturbed.
   for (int it = 0; it < 200000; ++it) {
     int64_t a[29] = {0x100000, 8 * 128, 128, 0x200000, 8 * 128, 128, 0x300000, 64, 0x400000, 8 * 16 * 128, 16 * 128,
@@ -143,6 +176,7 @@ int main() {
                            nullptr), "gather-perturbed");
   }
   fsk_set_option("xcd_skew", 3);
+  fsk_set_option("direct", 1);
   printf("done\n");
   return 0;
 }

@@ -13,6 +13,7 @@ from fasterkernels_amd import native as nat
 
 REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(REPO, "include", "fsk_decode.h")
+FSK_BOOL = 4  # a mask's type (fsk_decode_bounds, fsk_decode_dense_fp8)
 FAKE = 0x10000  # 64 KiB-aligned dummy address; never dereferenced on the host
 
 
@@ -67,11 +68,13 @@ def test_version_and_options(lib):
     assert lib.fsk_set_option(b"chunk_tokens", 0) == nat.FSK_OK
     assert lib.fsk_set_option(b"waves_per_cu", 0) == nat.FSK_ERR_INVALID
     assert lib.fsk_set_option(b"waves_per_cu", 8) == nat.FSK_OK
-    for name in (b"qk_engine", b"head_pairs"):
+    for name in (b"qk_engine", b"head_pairs", b"direct"):
         assert lib.fsk_set_option(name, 2) == nat.FSK_ERR_INVALID
         assert lib.fsk_set_option(name, -1) == nat.FSK_ERR_INVALID
     assert lib.fsk_set_option(b"qk_engine", 0) == nat.FSK_OK
     assert lib.fsk_set_option(b"head_pairs", 1) == nat.FSK_OK
+    for value in (0, 1):
+        assert lib.fsk_set_option(b"direct", value) == nat.FSK_OK
     for bad in (-1, 33, 288):  # a multiple of 32 in [0, 256]
         assert lib.fsk_set_option(b"seg_tokens", bad) == nat.FSK_ERR_INVALID
     for ok in (0, 256, 96):
@@ -228,6 +231,106 @@ def dense_fp8_args(**kw):
              wsb=1 << 30, chunk=0, stream=None)
     a.update(kw)
     return list(a.values())
+
+
+@pytest.mark.parametrize("override,code", [
+    (dict(q=None), nat.FSK_ERR_INVALID),
+    (dict(v=None), nat.FSK_ERR_INVALID),
+    (dict(out=None), nat.FSK_ERR_INVALID),
+    (dict(k=FAKE + 8), nat.FSK_ERR_INVALID),                   # not 16-byte aligned
+    (dict(q_n=0), nat.FSK_ERR_INVALID),
+    (dict(k_n=-1), nat.FSK_ERR_INVALID),
+    (dict(v_n=1 << 40), nat.FSK_ERR_UNSUPPORTED),
+    (dict(S=0), nat.FSK_ERR_INVALID),
+    (dict(S=1 << 31), nat.FSK_ERR_INVALID),
+    (dict(B=-1), nat.FSK_ERR_INVALID),
+    (dict(B=16385), nat.FSK_ERR_UNSUPPORTED),
+    (dict(Hkv=0), nat.FSK_ERR_INVALID),
+    (dict(Hq=30), nat.FSK_ERR_INVALID),
+    (dict(Hq=34, Hkv=2), nat.FSK_ERR_UNSUPPORTED),             # 17 query heads per KV head
+    (dict(D=96), nat.FSK_ERR_UNSUPPORTED),
+    (dict(dt=nat.FSK_F32), nat.FSK_ERR_UNSUPPORTED),
+    (dict(dt=nat.FSK_E4M3), nat.FSK_ERR_UNSUPPORTED),
+    (dict(odt=nat.FSK_E4M3), nat.FSK_ERR_UNSUPPORTED),
+    (dict(mdt=nat.FSK_E4M3), nat.FSK_ERR_UNSUPPORTED),
+    (dict(mdt=FSK_BOOL + 1), nat.FSK_ERR_UNSUPPORTED),
+    (dict(mask=FAKE + 1), nat.FSK_ERR_INVALID),                # bf16 at an odd address
+    (dict(m_ss=-1), nat.FSK_ERR_INVALID),
+    (dict(m_sb=1 << 40), nat.FSK_ERR_UNSUPPORTED),
+    (dict(position=FAKE), nat.FSK_ERR_INVALID),                # a mask, or a position and window
+    (dict(window=5), nat.FSK_ERR_INVALID),
+    (dict(k_st=120), nat.FSK_ERR_INVALID),                     # overlapping rows
+    (dict(k_st=1 << 26), nat.FSK_ERR_UNSUPPORTED),             # past the kernels' 32-bit offsets
+    (dict(chunk=48), nat.FSK_ERR_INVALID),
+    (dict(scale=float("inf")), nat.FSK_ERR_INVALID),
+    (dict(ws=None), nat.FSK_ERR_WORKSPACE),
+    (dict(ws=FAKE + 128), nat.FSK_ERR_WORKSPACE),
+    (dict(wsb=4096), nat.FSK_ERR_WORKSPACE),
+])
+def test_dense_fp8_validation(lib, override, code):
+    assert lib.fsk_decode_dense_fp8(*dense_fp8_args(**override)) == code
+    assert lib.fsk_last_error()
+
+
+def test_dense_fp8_workspace(lib):
+    """The dense call's workspace and, in front of it, the maxima and ranges:
+    a byte less is refused."""
+    shape = (4, 32, 8, 128, 512)
+    need = lib.fsk_decode_dense_fp8_workspace_bytes(*shape, 0)
+    dense = lib.fsk_workspace_bytes(nat.FSK_LAYOUT_DENSE, *shape, 16, 0)
+    assert need >= dense + 3 * 256 * 4 + 2 * 4 * 4
+    assert lib.fsk_decode_dense_fp8(*dense_fp8_args(wsb=need - 1)) == nat.FSK_ERR_WORKSPACE
+    for bad, code in (((-1, 32, 8, 128, 512, 0), nat.FSK_ERR_INVALID), ((4, 30, 8, 128, 512, 0), nat.FSK_ERR_INVALID),
+                      ((4, 32, 8, 96, 512, 0), nat.FSK_ERR_UNSUPPORTED), ((4, 32, 8, 128, -1, 0), nat.FSK_ERR_INVALID),
+                      ((4, 32, 8, 128, 512, 33), nat.FSK_ERR_INVALID)):
+        assert lib.fsk_decode_dense_fp8_workspace_bytes(*bad) == code
+
+
+def test_bounds_validation(lib):
+    ok = dict(mask=FAKE, dt=nat.FSK_F32, sb=512, ss=1, position=None, window=-1, B=4, S=512, ends=FAKE, starts=FAKE,
+              stream=None)
+    bare = dict(mask=None, starts=None)
+    for override, code in [
+            (dict(B=-1), nat.FSK_ERR_INVALID), (dict(S=0), nat.FSK_ERR_INVALID), (dict(S=-5), nat.FSK_ERR_INVALID),
+            (dict(B=16385), nat.FSK_ERR_UNSUPPORTED), (dict(ends=None), nat.FSK_ERR_INVALID),
+            (dict(starts=None), nat.FSK_ERR_INVALID), (dict(bare, window=0), nat.FSK_ERR_INVALID),
+            (dict(position=FAKE), nat.FSK_ERR_INVALID), (dict(window=0), nat.FSK_ERR_INVALID),
+            (dict(dt=nat.FSK_E4M3), nat.FSK_ERR_UNSUPPORTED), (dict(dt=-1), nat.FSK_ERR_UNSUPPORTED),
+            (dict(dt=FSK_BOOL + 1), nat.FSK_ERR_UNSUPPORTED), (dict(sb=-1), nat.FSK_ERR_INVALID),
+            (dict(ss=1 << 40), nat.FSK_ERR_UNSUPPORTED), (dict(mask=FAKE + 2), nat.FSK_ERR_INVALID)]:
+        assert lib.fsk_decode_bounds(*dict(ok, **override).values()) == code, override
+        assert lib.fsk_last_error()
+    assert lib.fsk_decode_bounds(*dict(ok, B=0).values()) == nat.FSK_OK  # nothing to do
+    assert lib.fsk_decode_bounds(*dict(ok, B=0, dt=FSK_BOOL, mask=FAKE + 1).values()) == nat.FSK_OK
+
+
+def test_quantize_validation(lib):
+    sizes = [lib.fsk_quantize_workspace_bytes(n) for n in range(5)]
+    assert sizes[0] == sizes[4] == nat.FSK_ERR_INVALID and 0 < sizes[1] < sizes[2] < sizes[3]
+
+    def call(count=3, src=(FAKE,) * 3, numel=(100,) * 3, dt=nat.FSK_F32, dst=(FAKE,) * 3, scale=(FAKE,) * 3, ws=FAKE,
+             wsb=1 << 20, null=None):
+        pointers = lambda x: ctypes.cast((ctypes.c_void_p * len(x))(*x), ctypes.c_void_p)  # noqa: E731
+        args = [pointers(src), ctypes.cast((ctypes.c_int64 * len(numel))(*numel), ctypes.c_void_p), dt, pointers(dst),
+                pointers(scale)]
+        if null is not None:
+            args[null] = None
+        return lib.fsk_quantize_e4m3(count, *args, ws, wsb, None)
+
+    for kw, code in [(dict(count=0), nat.FSK_ERR_INVALID), (dict(count=4), nat.FSK_ERR_INVALID),
+                     (dict(null=0), nat.FSK_ERR_INVALID), (dict(null=1), nat.FSK_ERR_INVALID),
+                     (dict(null=3), nat.FSK_ERR_INVALID), (dict(null=4), nat.FSK_ERR_INVALID),
+                     (dict(dt=nat.FSK_E4M3), nat.FSK_ERR_UNSUPPORTED), (dict(dt=FSK_BOOL), nat.FSK_ERR_UNSUPPORTED),
+                     (dict(numel=(100, 0, 100)), nat.FSK_ERR_INVALID), (dict(numel=(100, 100, -1)), nat.FSK_ERR_INVALID),
+                     (dict(numel=(1 << 40, 1, 1)), nat.FSK_ERR_UNSUPPORTED), (dict(src=(FAKE, None, FAKE)), nat.FSK_ERR_INVALID),
+                     (dict(dst=(FAKE, FAKE, None)), nat.FSK_ERR_INVALID), (dict(scale=(None, FAKE, FAKE)), nat.FSK_ERR_INVALID),
+                     (dict(src=(FAKE + 8, FAKE, FAKE)), nat.FSK_ERR_INVALID),
+                     (dict(dst=(FAKE, FAKE + 1, FAKE)), nat.FSK_ERR_INVALID),
+                     (dict(scale=(FAKE, FAKE, FAKE + 2)), nat.FSK_ERR_INVALID),
+                     (dict(ws=None), nat.FSK_ERR_WORKSPACE), (dict(ws=FAKE + 2), nat.FSK_ERR_WORKSPACE),
+                     (dict(wsb=11), nat.FSK_ERR_WORKSPACE)]:
+        assert call(**kw) == code, kw
+        assert lib.fsk_last_error()
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="fake pointers: the launches have to fail")

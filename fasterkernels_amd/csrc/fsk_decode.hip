@@ -2443,9 +2443,9 @@ __global__ __launch_bounds__(kWriteThreads) void kv_write_kernel(WriteParams p) 
 // launches for up to three tensors: every workgroup's |x| maximum, then the
 // codes.  HBM-bound: the source is read twice (the second time largely from
 // the 256 MB Infinity Cache) and the codes written once.  As torch operations
-// this was eight passes over fp32 copies: Q, K and V of 4 x 8 heads x 3827
-// tokens x 128 (bf16, 62.7 MB) in 24 launches, 259 us; the maxima take 13 us
-// and the codes 17 us (traced).  The attention hook's fp8 form does not store
+// this was eight passes over fp32 copies: Q, K and V of 4 x 8 heads x 4011
+// tokens x 128 (bf16, 65.7 MB) in 24 launches, 268 us; the maxima take 13.6 us
+// and the codes 16.5 us (traced).  The attention hook's fp8 form does not store
 // the codes at all (bounds_amax_kernel and the decode kernels' kQuant kinds).
 constexpr int kQuantMax = 3;         // tensors per call
 constexpr int kQuantThreads = 256;
@@ -2614,8 +2614,8 @@ __global__ __launch_bounds__(kQuantThreads) void quant_codes_kernel(QuantParams 
 // sequence reads its row (4 KB at 2048 positions of bf16) with 16-byte loads,
 // all in flight at once, and reduces it in registers.  As nine torch kernels
 // (compare, arange, two selects, two reductions over int32 rows, ...) the
-// range cost more than the attention: 4 left-padded sequences of up to 2047
-// positions, attention call 64.3 us (host-bound), with this 2.4 us launch 15.7.
+// range cost more than the attention: 4 left-padded sequences of up to 1468
+// positions, attention call 63 us (host-bound), with this 2.4 us launch 13.1.
 constexpr int kBoundsThreads = 256;
 constexpr int kBool = FSK_BOOL;
 struct BoundsParams {
@@ -2738,10 +2738,12 @@ __global__ __launch_bounds__(kBoundsThreads) void bounds_kernel(BoundsParams p) 
 // [0, p.blocks)) and the |x| maxima of Q, K and V, which do not depend on each
 // other.  The decode kernels take the scales from the maxima and quantise the
 // 16-bit rows between LDS and the matrix cores, so the codes are neither
-// written nor read: 4 x 8 heads x 3827 tokens x 128 bf16, ranges + maxima 12.6
-// us and the partial kernel 16.6 (16-bit rows alone 15, codes 10), against 2.6 +
-// 13 + 17 + 10 us with stored codes; the call 45.6 -> 31.8 us, and 26.5 -> 11.4
-// for one of 50 tokens (two launches instead of four).  The conversion is not
+// written nor read: 4 x 8 heads x 4011 tokens x 128 bf16, ranges + maxima 12.6
+// us and the partial kernel 16.6 (16-bit rows alone 14.1, codes 10), against 2.8
+// + 13.6 + 16.5 + 10 us with stored codes; the call 45.6 -> 31.5 us, and 26.5 ->
+// 11.4 for one of 50 tokens (two launches instead of four).  The results are
+// those of the stored codes: the split and the order of every sum are theirs
+// (on the split kernels; the direct kernel takes other sizes than theirs).  The conversion is not
 // what bounds it: an fp32 quotient of two FMAs instead of the binary64 one
 // measured the same 16.5 us, a branch around it for infinite scales 24 us (10K
 // instructions, with the clamp).

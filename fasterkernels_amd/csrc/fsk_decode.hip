@@ -2743,10 +2743,10 @@ __global__ __launch_bounds__(kBoundsThreads) void bounds_kernel(BoundsParams p) 
 // + 13.6 + 16.5 + 10 us with stored codes; the call 45.6 -> 31.5 us, and 26.5 ->
 // 11.4 for one of 50 tokens (two launches instead of four).  The results are
 // those of the stored codes: the split and the order of every sum are theirs
-// (on the split kernels; the direct kernel takes other sizes than theirs).  The conversion is not
-// what bounds it: an fp32 quotient of two FMAs instead of the binary64 one
-// measured the same 16.5 us, a branch around it for infinite scales 24 us (10K
-// instructions, with the clamp).
+// (on the split kernels; the direct kernel takes other sizes than theirs).  The
+// conversion is not what bounds it: an fp32 quotient of two FMAs instead of the
+// binary64 one measured the same 16.5 us, a branch around it for infinite scales
+// 24 us (10K instructions, with the clamp).
 template <int kSrc>
 __global__ __launch_bounds__(kQuantThreads) void bounds_amax_kernel(BoundsParams bp, QuantParams p) {
   static_assert(kQuantThreads == kBoundsThreads, "one workgroup size");
@@ -3317,8 +3317,8 @@ int dispatch_direct_layout(int layout, const DirectParams& dp, int waves, int q_
 // or four sequences of that length among ones of 16 tokens, and 16 tokens
 // throughout.  What the split kernels need for those grows with the workgroups
 // and with the query heads of each (rows to reduce): the lines move up with
-// groups x sqrt(query heads of a workgroup).  Measured at seven head shapes,
-// fp16 and e4m3, 64 to 4096 workgroups, extents of 128 to 1024 tokens and six
+// groups x sqrt(query heads of a workgroup).  Measured at nine head shapes,
+// fp16 and e4m3, 64 to 16384 workgroups, extents of 64 to 1024 tokens and six
 // mixes (replayed graphs, split against direct): 33 % off in the mean, 9 of
 // 8088 points over by more than 3 %, none by 5 %.  One line at 512 KB and 128
 // workgroups for every mix and up to 4 waves everywhere had 383 such points, up
@@ -3347,6 +3347,7 @@ struct DirectLine {
 };
 constexpr DirectLine kDirectLines[] = {{1536, 1024, 512, 384}, {768, 1024, 448, 384}, {512, 1024, 384, 384},
                                        {256, 896, 320, 256},   {128, 896, 256, 256},  {0, 768, 192, 64}};
+static_assert(kDirectLines[0].tokens <= kDirectTokens, "the page windows hold the longest direct call");
 int direct_waves(const Common& c, int64_t groups, bool pair) {
   if (!g_opt.direct || c.chunk > 0 || g_opt.chunk_tokens > 0 || g_opt.qk_engine != 0) return 0;
   const int64_t extent = c.layout == FSK_LAYOUT_PAGED ? c.kv_extent * c.page_size : c.kv_extent;

@@ -3317,12 +3317,14 @@ int dispatch_direct_layout(int layout, const DirectParams& dp, int waves, int q_
 // or four sequences of that length among ones of 16 tokens, and 16 tokens
 // throughout.  What the split kernels need for those grows with the workgroups
 // and with the query heads of each (rows to reduce): the lines move up with
-// groups x sqrt(query heads of a workgroup).  Measured at nine head shapes,
-// fp16 and e4m3, 64 to 16384 workgroups, extents of 64 to 1024 tokens and six
-// mixes (replayed graphs, split against direct): 33 % off in the mean, 9 of
-// 8088 points over by more than 3 %, none by 5 %.  One line at 512 KB and 128
-// workgroups for every mix and up to 4 waves everywhere had 383 such points, up
-// to 78 %.  us, split -> direct, 8 KV heads x 128 of fp16, 32 query heads: 1 x
+// groups x sqrt(query heads of a workgroup).  (Just past 256 workgroups some CUs
+// hold two long ones and others one: 40 x U[1,768] bf16, 8 KV heads x 128, 16.9 us
+// split, 19.2 direct; so up to 400 no more than 320 KB.)  Measured at 14 head
+// shapes, fp16, bf16 and e4m3, 64 to 16384 workgroups, extents of 64 to 1024
+// tokens and six mixes (replayed graphs, split against direct): 30 % off in the
+// mean, 19 of 12323 points over by more than 3 %, the worst 7 %.  One line at 512
+// KB and 128 workgroups for every mix and up to 4 waves everywhere had 560 such
+// points, up to 78 %.  us, split -> direct, 8 KV heads x 128 of fp16, 32 query heads: 1 x
 // 64 tokens 8.4 -> 4.5, 1 x 384 8.4 -> 6.9, 16 x 512 11.1 -> 8.9 (one of 512
 // among 15 of 16: 8.8 -> 7.6), 64 x 256 16.2 -> 12.4, 64 x 896 40.7 -> 36.4 (one:
 // 11.4 -> 10.6), 256 x 64 23.7 -> 12.9, 256 x U[1,1024] 98.6 -> 83.4; past the
@@ -3345,7 +3347,7 @@ struct DirectLine {
   int tokens;       // longest extent
   int kb, kb_d256;  // ... and its K/V of a head: 16-bit rows of head_dim 256 (kb_d256), others
 };
-constexpr DirectLine kDirectLines[] = {{1536, 1024, 512, 384}, {768, 1024, 448, 384}, {512, 1024, 384, 384},
+constexpr DirectLine kDirectLines[] = {{1536, 1024, 512, 384}, {1024, 1024, 448, 384}, {512, 1024, 384, 384},
                                        {256, 896, 320, 256},   {128, 896, 256, 256},  {0, 768, 192, 64}};
 static_assert(kDirectLines[0].tokens <= kDirectTokens, "the page windows hold the longest direct call");
 int direct_waves(const Common& c, int64_t groups, bool pair) {
@@ -3359,7 +3361,9 @@ int direct_waves(const Common& c, int64_t groups, bool pair) {
   while (level < line->level) ++line;
   int64_t row = 2 * (int64_t)c.D * elem_bytes(c.kv_dt);  // K/V bytes of a token and head
   if (pair || c.pre) row = row * 3 / 2;
-  if (extent > line->tokens || extent * row > (c.D == 256 && !e4m3 ? line->kb_d256 : line->kb) * 1024) return 0;
+  int kb = c.D == 256 && !e4m3 ? line->kb_d256 : line->kb;
+  if (groups > 256 && groups <= 400) kb = std::min(kb, 320);
+  if (extent > line->tokens || extent * row > kb * 1024) return 0;
   const int64_t tiles = cdiv(extent, 32);
   const int64_t two = (heads >= 4 ? 3072 : 2048) * (e4m3 || c.D == 64 ? 3 : 2) / 2;
   const int64_t most = groups <= 16 || (e4m3 && groups <= 256 && extent > 2 * groups) ? kDirectMaxWaves

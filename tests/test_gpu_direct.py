@@ -152,7 +152,8 @@ def test_block_scores(layout, out, mode, option):
 @pytest.mark.parametrize("kv,Hq,B,longest,direct", [
     ("f16", 32, 1, 384, 1), ("f16", 32, 1, 385, 0), ("f16", 32, 15, 384, 1), ("f16", 32, 15, 1024, 0),
     ("f16", 32, 16, 640, 1), ("f16", 32, 16, 641, 0), ("f16", 32, 32, 768, 1), ("f16", 32, 32, 769, 0),
-    ("f16", 32, 48, 896, 1), ("f16", 32, 48, 897, 0), ("f16", 32, 96, 1024, 1), ("f16", 32, 96, 1025, 0),
+    ("f16", 32, 48, 640, 1), ("f16", 32, 48, 641, 0), ("f16", 32, 51, 768, 1), ("f16", 32, 64, 896, 1),
+    ("f16", 32, 64, 897, 0), ("f16", 32, 96, 1024, 1), ("f16", 32, 96, 1025, 0),
     ("f16", 8, 16, 512, 1), ("f16", 8, 16, 513, 0), ("f16", 8, 192, 1024, 1), ("f16", 8, 191, 1024, 0),
     ("f16", 32, 300, 100, 1), ("e4m3", 32, 1, 768, 1), ("e4m3", 32, 2, 769, 0), ("e4m3", 32, 20, 896, 1),
     ("e4m3", 32, 20, 897, 0), ("e4m3", 32, 32, 1024, 1), ("e4m3", 32, 32, 1025, 0)])
